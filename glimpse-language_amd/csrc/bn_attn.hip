@@ -19,7 +19,7 @@
 #include "bn_prefill_pair.h"
 #include "bn_prep.h"
 #include "bn_ternary.h"
-#include "bn_ternary_pf.h"
+#include "bn_ternary_mx.h"
 #include "bn_util_kernels.h"
 #include "bn_verify.h"
 
@@ -918,44 +918,49 @@ bn_status run_ternary(bn_ctx* ctx, hipStream_t st, const bn_ternary_args* a) {
         const dim3 grid((unsigned)row_tiles);
         // fewer 64-row tiles than CUs (o_proj-sized matrices): 8 waves per block split K further
         if (row_tiles < ctx->cus && a->k % (8 * bn::TERN_KC) == 0)
-            bn_launch(ctx, (bn::tern_mfma_kernel<1, 8, 1>), grid, dim3(512), 0, st, t, row_tiles);
+            bn_launch(ctx, (bn::tern_mfma_kernel<8>), grid, dim3(512), 0, st, t, row_tiles);
         else if (tern_ksplit(a->k) == 4)
-            bn_launch(ctx, (bn::tern_mfma_kernel<1, 4, 1>), grid, dim3(256), 0, st, t, row_tiles);
+            bn_launch(ctx, (bn::tern_mfma_kernel<4>), grid, dim3(256), 0, st, t, row_tiles);
         else
-            bn_launch(ctx, (bn::tern_mfma_kernel<1, 2, 1>), grid, dim3(128), 0, st, t, row_tiles);
-        return launched(ctx, "tern_mfma_kernel<1>");
+            bn_launch(ctx, (bn::tern_mfma_kernel<2>), grid, dim3(128), 0, st, t, row_tiles);
+        return launched(ctx, "tern_mfma_kernel");
     }
-    bool split_once = a->work != nullptr && bn::tern_pf_tiles((int)a->T, (int)a->k) <= (size_t)INT32_MAX;
-    for (uint32_t i = 0; i < a->n_mats; ++i) split_once = split_once && !((uintptr_t)a->mat[i].s & 3);
-    if (split_once) {
-        // x split once into the workspace, then the GEMM streams it
-        const size_t tiles = bn::tern_pf_tiles((int)a->T, (int)a->k);
-        uint8_t* work = static_cast<uint8_t*>(a->work);
-        bn_launch(ctx, bn::tern_split_kernel, dim3((unsigned)tiles), dim3(256), 0, st, a->x, a->x_ts, (int)a->T,
-                           (int)a->k, work);
-        const int row_tiles = (int)ceil_div(rows, 256);
-        const int64_t blocks = (int64_t)row_tiles * ceil_div(a->T, bn::TPF_BM);
-        if (blocks > INT32_MAX) return set_err(ctx->err, BN_EINVAL, "T * rows too large for one launch");
-        // a grid of 64-token blocks that fits three per CU in one round runs as such (2 copy stages, three blocks
-        // per CU); a larger one takes 128-token blocks (each decoded weight feeds twice the MFMAs; 2 stages, two
-        // blocks per CU): the 4B q/k/v projection over 4,096 tokens 426-437 -> 387-405 us, same results bit for bit
-        if (blocks <= 3 * (int64_t)ctx->cus)
-            bn_launch(ctx, (bn::tern_pf_kernel<2, 3, 2>), dim3((unsigned)blocks), dim3(256), 0, st, t, row_tiles,
-                               (const uint8_t*)work);
+    // x's digits once per call into the workspace, or made by every block (the same products in the same order).
+    // Blocks by the tiles a call gives (measured, us, 2B q/k/v, 2B o, 4B q/k/v, 4B o_proj rows):
+    //  - 32 tokens x 128 rows, the columns split over two wave groups, up to 1.5 such blocks per CU: a step is bound by
+    //    the latencies of its copies and operand reads, and two groups take half the steps (33 tokens: 16.4, 19.4,
+    //    19.1, 32.8 against 22.2, 25.0, 26.1, 43.2 unsplit; 640 blocks, 4B q/k/v of 250 tokens: 38.7 against 37.0)
+    //  - 32 x 256 up to two per CU (their two stages let three stay on a CU; 4B o_proj of 1,017 tokens: 64.4 against
+    //    74.4 with 64 x 256, of 2,000: 114 against 104)
+    //  - 64 x 256 beyond: each decoded weight feeds twice the MFMAs
+    // Without a workspace every block makes its own digits, vector work that twice the rows halve: 64 x 512 where such
+    // blocks fill their rounds over the CUs (4B q/k/v of 4,096 tokens: 387 against 410; of 1,017: 151 against 133).
+    const int64_t dig_blocks = ceil_div(a->T, 64) * (int64_t)(a->k / bn::TMX_G);
+    const int64_t small = ceil_div(a->T, 32) * ceil_div(rows, 128), mid = ceil_div(a->T, 32) * ceil_div(rows, 256);
+    const int64_t large = ceil_div(a->T, 64) * ceil_div(rows, 256);
+    const int64_t cus = ctx->cus, large8 = ceil_div(a->T, 64) * ceil_div(rows, 512);
+    const bool split = 2 * small <= 3 * cus;
+    if (large > INT32_MAX) return set_err(ctx->err, BN_EINVAL, "T * rows too large for one launch");
+    const uint8_t* work = static_cast<const uint8_t*>(a->work);
+    const int rt128 = (int)ceil_div(rows, 128), rt256 = (int)ceil_div(rows, 256);
+    if (work && dig_blocks <= INT32_MAX) {
+        bn_launch(ctx, bn::tern_digits_kernel, dim3((unsigned)dig_blocks), dim3(256), 0, st, a->x, a->x_ts, (int)a->T,
+                  (int)a->k, static_cast<uint8_t*>(a->work));
+        if (split)
+            bn_launch(ctx, (bn::tern_mx_kernel<2, 1, 2, true>), dim3((unsigned)small), dim3(256), 0, st, t, rt128, work);
+        else if (mid <= 2 * cus)
+            bn_launch(ctx, (bn::tern_mx_kernel<4, 1, 1, true>), dim3((unsigned)mid), dim3(256), 0, st, t, rt256, work);
         else
-            bn_launch(ctx, (bn::tern_pf_kernel<2, 2, 4>),
-                      dim3((unsigned)(row_tiles * ceil_div(a->T, 2 * bn::TPF_BM))), dim3(256), 0, st, t, row_tiles,
-                      (const uint8_t*)work);
-        return launched(ctx, "tern_pf_kernel");
+            bn_launch(ctx, (bn::tern_mx_kernel<4, 2, 1, true>), dim3((unsigned)large), dim3(256), 0, st, t, rt256, work);
+    } else if (split) {
+        bn_launch(ctx, (bn::tern_mx_kernel<2, 1, 2, false>), dim3((unsigned)small), dim3(256), 0, st, t, rt128, work);
+    } else if (8 * large8 >= 6 * cus * ceil_div(large8, cus)) {
+        bn_launch(ctx, (bn::tern_mx_kernel<8, 2, 1, false>), dim3((unsigned)large8), dim3(512), 0, st, t,
+                  (int)ceil_div(rows, 512), work);
+    } else {
+        bn_launch(ctx, (bn::tern_mx_kernel<4, 2, 1, false>), dim3((unsigned)large), dim3(256), 0, st, t, rt256, work);
     }
-    constexpr int MT = BN_TERN_PF_MT;
-    constexpr int RG = BN_TERN_PF_RG;
-    const int row_tiles = (int)ceil_div(rows, 64 * RG);
-    const int64_t blocks = (int64_t)row_tiles * ceil_div(a->T, 32 * MT);
-    if (blocks > INT32_MAX) return set_err(ctx->err, BN_EINVAL, "T * rows too large for one launch");
-    bn_launch(ctx, (bn::tern_mfma_kernel<MT, 1, RG, BN_TERN_PF_OCC, BN_TERN_PF_KC>), dim3((unsigned)blocks),
-                       dim3(64 * RG), 0, st, t, row_tiles);
-    return launched(ctx, "tern_mfma_kernel (prefill)");
+    return launched(ctx, "tern_mx_kernel");
 }
 
 // The LoRA-A rows of an attention call, after it (a->lora_r > 0): lora_kernel rebuilds the gated rows from `out`.

@@ -5,10 +5,10 @@
 // Weight format (kernels/qmv.glsl:1-2): row n of W is K/16 uint32 words, word j holding codes of k = 16j + e at
 // bits [2e, 2e+2); one fp16 scale per 128 codes, s[n * K/128 + k/128]; weight = scale * (code - 1).
 //
-// Two kernels:
+// Kernels:
 //   tern_rows_kernel<NT> (T <= 4): VALU. Lanes take words of 8 rows at a time; per word and token the reference's
 //     decode arithmetic, acc += s * (sum_e x_e * code_e - sum_e x_e) (qmv.glsl:22-35), then a wave sum.
-//   tern_mfma_kernel<MT, KS> (T > 4): v_mfma_f32_32x32x16_f16 with X as A (tokens) and W as B (rows). Weights are
+//   tern_mfma_kernel<KS> (T = 5..32): v_mfma_f32_32x32x16_f16 with X as A (tokens) and W as B (rows). Weights are
 //     exact in fp16 ((code - 1) * scale is -s, 0, s or 2s); X is split into hi = fp16(x) rounded toward zero and
 //     lo = fp16(x - hi), two MFMAs per tile, so each product carries 22 of x's 24 mantissa bits and every sum is
 //     fp32: the same result class as the reference's fp32 matmuls (qmm3.comp, the Metal qmm's float MMA), not an
@@ -19,8 +19,7 @@
 //     such a token included) keeps about 22 bits; the check costs one compare per value.
 //     Codes become fp16 weights through v_perm_b32 on a per-row 8-byte table of -s, 0, s, 2s (no conversion or
 //     multiply per code).
-//   tern_split_kernel + tern_pf_kernel (T > 32 with a workspace, bn_ternary_pf.h): the same arithmetic with x split
-//     once per call.
+//   tern_digits_kernel + tern_mx_kernel (T > 32, bn_ternary_mx.h): fp6 x fp4 MFMAs over base-32 digits of x.
 // All write y = (add ? y + v : v) + sum_j u[j] * B[n, j] (store_post, qmv.glsl:10-15).
 #pragma once
 #include "bn_device.h"
@@ -200,20 +199,6 @@ __global__ __launch_bounds__(256) void tern_rows_kernel(TernArgs a) {
 
 // ---- MFMA kernel --------------------------------------------------------------------------------------------
 constexpr int TERN_KC = 64;  // k per staged chunk (4 MFMA k-steps of 16)
-// prefill kernel shape: 32-token tiles per wave and waves per SIMD it is compiled for
-#ifndef BN_TERN_PF_MT
-#define BN_TERN_PF_MT 2
-#endif
-#ifndef BN_TERN_PF_OCC
-#define BN_TERN_PF_OCC 3
-#endif
-#ifndef BN_TERN_PF_RG
-#define BN_TERN_PF_RG 4
-#endif
-#ifndef BN_TERN_PF_KC
-#define BN_TERN_PF_KC 64
-#endif
-
 // The four weights (code - 1) * s of one row and scale group as a v_perm_b32 table: lo holds the low bytes of the
 // fp16 entries for codes 0..3 (-s, 0, s, 2s), hi their high bytes. 2s = s + s is exact wherever (code - 1) * s is
 // finite in fp16.
@@ -247,28 +232,19 @@ __device__ __forceinline__ h8 tern_decode8(uint32_t w, uint32_t dup, TernTab t) 
     return r;
 }
 
-// A block whose waves each stage their own K range (KS > 1, one row group) orders its LDS writes and reads within
-// the wave (LDS instructions of one wave complete in order); a block whose waves share the staged tile syncs.
-template <int KS>
+// The waves stage their own K ranges: LDS writes and reads are ordered within the wave (LDS instructions of one wave
+// complete in order).
 __device__ __forceinline__ void tern_sync() {
-    if constexpr (KS > 1) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    } else {
-        __syncthreads();
-    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // LDS row of token row m in block k = 2q + kg of a staged chunk: m XOR a per-block mask, a bijection inside each
 // 16-row group. Staging writes 8 (or 16) consecutive lanes to the same m in consecutive blocks, which start BM * 16
 // bytes apart (the same banks); the mask spreads them over distinct 16-byte bank slots, and the A-operand reads
 // (32 consecutive m per block) stay a permutation of slots within every 8- and 16-lane group.
-template <int NQ>
-__device__ __forceinline__ int tern_swz(int m, int k) {
-    if constexpr (NQ == 4) return m ^ (k | ((m & 1) << 3));
-    else return m ^ (k & 15);
-}
+__device__ __forceinline__ int tern_swz(int m, int k) { return m ^ (k | ((m & 1) << 3)); }
 
 #ifndef BN_TERN_XCD_GROUP
 #define BN_TERN_XCD_GROUP 4
@@ -276,8 +252,7 @@ __device__ __forceinline__ int tern_swz(int m, int k) {
 
 // Block -> (row tile rt, token tile tt). Workgroups are dealt to the 8 XCDs round robin (block b on XCD b % 8), and
 // each XCD has its own L2. When the token tiles divide evenly, XCD x takes the token tiles x, x + 8, ... in groups of
-// G (BN_TERN_XCD_GROUP by default; tern_pf_kernel's 128-token blocks take half as many, so a group spans the same
-// tokens) and runs every row tile of a group before the next group, the group's token tiles of one row tile on
+// G (BN_TERN_XCD_GROUP for 64-token blocks, as many tokens for others) and runs every row tile of a group before the next group, the group's token tiles of one row tile on
 // consecutive blocks: each x tile is fetched into one L2 (and stays there while the row tiles pass), and each row
 // tile's codes serve the group from that L2. Otherwise row tiles run fastest (token tile by token tile).
 template <int BM, int G = BN_TERN_XCD_GROUP>
@@ -358,48 +333,37 @@ __device__ __forceinline__ void tern_absmax8(float& mx, f4 va, f4 vb) {
     for (int s = 0; s < 4; ++s) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(mx) : "v"(va[s]), "v"(vb[s]));
 }
 
-// MT 32-token tiles x 2 32-row tiles per wave; KS waves split K (their partial sums meet in LDS in ks order), RG
-// waves split rows (KS > 1 only with RG = 1). Block: 64 * KS * RG threads, 32 * MT tokens x 64 * RG rows.
+// One 32-token tile x 2 32-row tiles per wave; KS waves split K (their partial sums meet in LDS in ks order). Block:
+// 64 KS threads, 32 tokens x 64 rows.
 //
-// A layout in LDS, per k-split group: hi[KC / 16 q][2 kg][32 MT m][8 slots] fp16, then lo the same. Slot i of (q, kg, m)
+// A layout in LDS, per wave: hi[KC / 16 q][2 kg][32 m][8 slots] fp16, then lo the same. Slot i of (q, kg, m)
 // holds x[m][k0 + 16q + 4kg + 8(i & 1) + (i >> 1)], the k order tern_decode8 gives the B operand, so each lane's A
 // operand (m = lane % 32, kg = lane / 32) is one 16-byte LDS read.
-template <int MT, int KS, int RG, int OCC = 1, int KC = TERN_KC>
-__global__ __launch_bounds__(64 * KS * RG, OCC) void tern_mfma_kernel(TernArgs a, int row_tiles) {
-    constexpr int NQ = KC / 16;        // MFMA k-steps per chunk
-    static_assert(KC == 64 || KC == 128, "a chunk lies inside one 128-column scale group");
-    static_assert(KS * RG <= 8 && (KS == 1 || (RG == 1 && MT == 1)), "split-K blocks are one token tile, one row group");
-    constexpr int BM = 32 * MT;        // tokens per block
-    constexpr int GROUP_H = 2 * NQ * 2 * BM * 8;  // fp16 per k-split group (hi and lo): NQ q * 2 kg * BM * 8 * 2
-    // one buffer, two syncs per chunk: a second buffer costs registers and occupancy (3 -> 2 waves per SIMD for
-    // the prefill shape) and measured slower on MI355X
+template <int KS>
+__global__ __launch_bounds__(64 * KS, 1) void tern_mfma_kernel(TernArgs a, int row_tiles) {
+    constexpr int KC = TERN_KC, NQ = KC / 16;     // MFMA k-steps per chunk
+    static_assert(KS == 2 || KS == 4 || KS == 8, "waves per block");
+    constexpr int BM = 32;                        // tokens per block
+    constexpr int GROUP_H = 2 * NQ * 2 * BM * 8;  // fp16 per wave (hi and lo): NQ q * 2 kg * BM * 8 * 2
     __shared__ __attribute__((aligned(16))) _Float16 lds[KS * GROUP_H];
-    // per wave (KS = 1): whether it staged a token with a value >= TERN_BIG in the current chunk. Written before and read
-    // after the chunk's staging barrier; the next chunk writes only after the barrier that opens it, which every
-    // wave reaches after its reads.
-    __shared__ __attribute__((aligned(16))) int big_flag[KS == 1 ? RG : 1];
     static_assert(KS * GROUP_H * 2 <= 65536, "LDS");
-    static_assert(KS * 32 * MT * 64 * 4 <= KS * GROUP_H * 2 || KS == 1, "reduction buffer fits the A buffer");
+    static_assert(KS * 32 * 64 * 4 <= KS * GROUP_H * 2, "reduction buffer fits the A buffer");
 
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int rg = wave / KS, ks = wave % KS;
+    const int lane = threadIdx.x & 63, ks = threadIdx.x >> 6;
     int rt, tt;
     tern_tile<BM>((int)blockIdx.x, row_tiles, a.T, rt, tt);
     const int t0 = tt * BM;
-    const int rbase_g = (rt * RG + rg) * 64;  // first global row of this wave
-    const bool active = rbase_g < a.rows;
-    int rbase = active ? rbase_g : 0;
+    int rbase = rt * 64;  // first global row of this block (rows is a multiple of 64)
     const int mi = tern_member(a, rbase);
     const TernMat m = tern_mat(a, mi);
 
     const int K = a.K, kw = K >> 4, kg = K >> 7;
     const int klen = K / KS, kbase = ks * klen, nchunk = klen / KC;
 
-    // staging: group thread gt of 64 * RG takes units u = gt + i * 64 * RG, u = (m * NQ + q) * 2 + kgu; the 2 NQ
-    // units of one token in a chunk sit on 2 NQ consecutive lanes of the same i
-    constexpr int GT = 64 * RG, UPT = 2 * NQ * BM / GT;
-    static_assert(GT % (2 * NQ) == 0, "a token's units stay inside one wave");
-    const int gt = rg * 64 + lane;
+    // staging: lane gt takes units u = gt + i * 64, u = (m * NQ + q) * 2 + kgu; the 2 NQ units of one token in a chunk
+    // sit on 2 NQ consecutive lanes of the same i
+    constexpr int GT = 64, UPT = 2 * NQ * BM / GT;
+    const int gt = lane;
     _Float16* glds = lds + ks * GROUP_H;
     f4 xa[UPT], xb[UPT];
     auto load_x = [&](int c) __attribute__((always_inline)) {
@@ -407,12 +371,9 @@ __global__ __launch_bounds__(64 * KS * RG, OCC) void tern_mfma_kernel(TernArgs a
         for (int i = 0; i < UPT; ++i) {
             const int u = gt + i * GT;
             const int mm = u / (2 * NQ), q = (u >> 1) % NQ, kgu = u & 1;
-            // token rows past T are not staged: their A rows only feed outputs that are not stored. Prefill blocks
-            // (KS = 1) load them anyway from row T - 1 (in bounds), so that the next chunk's loads are unconditional
-            // and stay in flight (a conditional load leaves register copies that the compiler waits for right after
-            // issuing the next loads); split-K blocks of a few tokens skip them.
-            if (KS == 1 || t0 + mm < a.T) {
-                const float* p = a.x + (int64_t)min(t0 + mm, a.T - 1) * a.x_ts + kbase + c * KC + 16 * q + 4 * kgu;
+            // token rows past T are not staged: their A rows only feed outputs that are not stored
+            if (t0 + mm < a.T) {
+                const float* p = a.x + (int64_t)(t0 + mm) * a.x_ts + kbase + c * KC + 16 * q + 4 * kgu;
                 xa[i] = *reinterpret_cast<const f4*>(p);
                 xb[i] = *reinterpret_cast<const f4*>(p + 8);
             }
@@ -421,7 +382,7 @@ __global__ __launch_bounds__(64 * KS * RG, OCC) void tern_mfma_kernel(TernArgs a
     auto stage_unit = [&](int mm, int q, int kgu, f4 va, f4 vb, int mode) __attribute__((always_inline)) {
         h8 hi, lo;
         tern_split8(va, vb, mode, hi, lo);
-        const int off = ((q * 2 + kgu) * BM + tern_swz<NQ>(mm, q * 2 + kgu)) * 8;
+        const int off = ((q * 2 + kgu) * BM + tern_swz(mm, q * 2 + kgu)) * 8;
         *reinterpret_cast<h8*>(glds + off) = hi;
         *reinterpret_cast<h8*>(glds + 2 * NQ * BM * 8 + off) = lo;
     };
@@ -431,8 +392,7 @@ __global__ __launch_bounds__(64 * KS * RG, OCC) void tern_mfma_kernel(TernArgs a
         float mx = 0.0f;
 #pragma unroll
         for (int i = 0; i < UPT; ++i) tern_absmax8(mx, xa[i], xb[i]);
-        // the common case, no such value in any unit of the wave (a unit past T, which KS = 1 loads from row T - 1,
-        // can only send the wave to the general path below)
+        // the common case, no such value in any unit of the wave
         if (__ballot(mx >= TERN_BIG) == 0) {
 #pragma unroll
             for (int i = 0; i < UPT; ++i) {
@@ -489,20 +449,18 @@ __global__ __launch_bounds__(64 * KS * RG, OCC) void tern_mfma_kernel(TernArgs a
         }
     };
 
-    f16x acc[MT][2];
+    f16x acc[2];
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][nt][e] = 0.0f;
+        for (int e = 0; e < 16; ++e) acc[nt][e] = 0.0f;
 
     const uint32_t dup = kgl ? 0x03030101u : 0x02020000u;
     // inactive waves (rows past the last matrix) load member 0's first rows, in bounds, and do not use them
     load_x(0);
     load_w(0);
     for (int c = 0; c < nchunk; ++c) {
-        tern_sync<KS>();  // the previous chunk's A reads are done
+        tern_sync();  // the previous chunk's A reads are done
         const bool staged_big = store_x();
         u4 wcur[2][NQ / 4];
 #pragma unroll
@@ -518,25 +476,12 @@ __global__ __launch_bounds__(64 * KS * RG, OCC) void tern_mfma_kernel(TernArgs a
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) tab[nt] = tern_table(sv_next[nt]);
         asm volatile("" ::"v"(tab[0].lo), "v"(tab[0].hi), "v"(tab[1].lo), "v"(tab[1].hi));
-        // the staging is complete (block-wide for KS = 1, where the waves share it; wave-wide otherwise), and
-        // whether any token of it was held back for the scaled pass
-        bool chunk_big;
-        if constexpr (KS > 1) {
-            tern_sync<KS>();
-            chunk_big = __ballot(staged_big) != 0;
-        } else {
-            const bool wave_big = __ballot(staged_big) != 0;
-            if (lane == 0) big_flag[rg] = wave_big;
-            __syncthreads();
-            int f = 0;
-#pragma unroll
-            for (int r = 0; r < RG; ++r) f |= big_flag[r];
-            chunk_big = f != 0;
-        }
-        if (KS == 1 || c + 1 < nchunk) {
-            const int cn = min(c + 1, nchunk - 1);  // prefill blocks: the last chunk reloads itself (unused)
-            load_x(cn);
-            load_w(cn);
+        // the staging is complete, and whether any token of it was held back for the scaled pass
+        tern_sync();
+        const bool chunk_big = __ballot(staged_big) != 0;
+        if (c + 1 < nchunk) {
+            load_x(c + 1);
+            load_w(c + 1);
         }
         // the chunk's MFMAs over the staged hi/lo tiles
         auto mfma_chunk = [&](const u4 (&wc)[2][NQ / 4], const TernTab (&tb)[2]) __attribute__((always_inline)) {
@@ -545,32 +490,24 @@ __global__ __launch_bounds__(64 * KS * RG, OCC) void tern_mfma_kernel(TernArgs a
                 h8 b[2];
 #pragma unroll
                 for (int nt = 0; nt < 2; ++nt) b[nt] = tern_decode8(wc[nt][q >> 2][q & 3], dup, tb[nt]);
-                h8 ah[MT], al[MT];
+                const int off = ((q * 2 + kgl) * BM + tern_swz(n, q * 2 + kgl)) * 8;
+                const h8 ah = *reinterpret_cast<const h8*>(glds + off);
+                const h8 al = *reinterpret_cast<const h8*>(glds + 2 * NQ * BM * 8 + off);
 #pragma unroll
-                for (int i = 0; i < MT; ++i) {
-                    const int off = ((q * 2 + kgl) * BM + tern_swz<NQ>(32 * i + n, q * 2 + kgl)) * 8;
-                    ah[i] = *reinterpret_cast<const h8*>(glds + off);
-                    al[i] = *reinterpret_cast<const h8*>(glds + 2 * NQ * BM * 8 + off);
-                }
+                for (int nt = 0; nt < 2; ++nt) acc[nt] = mfma32(ah, b[nt], acc[nt]);
 #pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int nt = 0; nt < 2; ++nt) acc[i][nt] = mfma32(ah[i], b[nt], acc[i][nt]);
-#pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int nt = 0; nt < 2; ++nt) acc[i][nt] = mfma32(al[i], b[nt], acc[i][nt]);
+                for (int nt = 0; nt < 2; ++nt) acc[nt] = mfma32(al, b[nt], acc[nt]);
             }
         };
-        if (active) mfma_chunk(wcur, tab);
+        mfma_chunk(wcur, tab);
         if (chunk_big) {
             // rare: some token had a value beyond fp16's range in this chunk (decided uniformly for the threads that
             // share the staging). Its x, times 2^-16, is multiplied into acc times 2^-16, and acc is scaled back:
             // acc + 2^16 (x 2^-16) W^T, with every scaling a power of two (exact).
-            tern_sync<KS>();
+            tern_sync();
             store_big(c);
-            tern_sync<KS>();
-            if (active) {
+            tern_sync();
+            {
                 // the chunk's codes and scales again (the staged copies are not kept alive for this rare pass)
                 u4 wr[2][NQ / 4];
                 TernTab tr[2];
@@ -581,51 +518,33 @@ __global__ __launch_bounds__(64 * KS * RG, OCC) void tern_mfma_kernel(TernArgs a
                     tr[nt] = tern_table(srow[nt][(kbase + c * KC) >> 7]);
                 }
 #pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int nt = 0; nt < 2; ++nt) acc[i][nt] *= 1.0f / 65536.0f;
+                for (int nt = 0; nt < 2; ++nt) acc[nt] *= 1.0f / 65536.0f;
                 mfma_chunk(wr, tr);
 #pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int nt = 0; nt < 2; ++nt) acc[i][nt] *= 65536.0f;
+                for (int nt = 0; nt < 2; ++nt) acc[nt] *= 65536.0f;
             }
         }
     }
 
-    // C layout: acc[i][nt][j] = (token 32 i + 8 (j / 4) + 4 (lane / 32) + j % 4, row 32 nt + lane % 32)
-    if constexpr (KS == 1) {
-        if (!active) return;
+    // C layout: acc[nt][j] = (token 8 (j / 4) + 4 (lane / 32) + j % 4, row 32 nt + lane % 32)
+    // partial tiles of the KS waves: red[ks][32 tokens][64 rows]
+    float* red = reinterpret_cast<float*>(lds);
+    __syncthreads();
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
+    for (int j = 0; j < 16; ++j) {
+        const int tl = 8 * (j >> 2) + 4 * kgl + (j & 3);
 #pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const int t = t0 + 32 * i + 8 * (j >> 2) + 4 * kgl + (j & 3);
-                if (t < a.T)
+        for (int nt = 0; nt < 2; ++nt) red[(ks * 32 + tl) * 64 + 32 * nt + n] = acc[nt][j];
+    }
+    __syncthreads();
+    // thread p sums outputs p, p + 64 KS, ... of the 32 x 64 tile in ks order
+    for (int p = threadIdx.x; p < 32 * 64; p += 64 * KS) {
+        const int tl = p >> 6, col = p & 63;
+        if (t0 + tl >= a.T) continue;
+        float v = red[p];
 #pragma unroll
-                    for (int nt = 0; nt < 2; ++nt) tern_store(a, m, mi, t, rbase + 32 * nt + n, acc[i][nt][j]);
-            }
-    } else {
-        // partial tiles of the KS waves (one row group, MT = 1): red[ks][32 tokens][64 rows]
-        float* red = reinterpret_cast<float*>(lds);
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int tl = 8 * (j >> 2) + 4 * kgl + (j & 3);
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt) red[(ks * 32 + tl) * 64 + 32 * nt + n] = acc[0][nt][j];
-        }
-        __syncthreads();
-        if (!active) return;
-        // thread p sums outputs p, p + 256, ... of the 32 x 64 tile in ks order
-        for (int p = threadIdx.x; p < 32 * 64; p += 64 * KS) {
-            const int tl = p >> 6, col = p & 63;
-            if (t0 + tl >= a.T) continue;
-            float v = red[p];
-#pragma unroll
-            for (int k2 = 1; k2 < KS; ++k2) v += red[k2 * 32 * 64 + p];
-            tern_store(a, m, mi, t0 + tl, rbase + col, v);
-        }
+        for (int k2 = 1; k2 < KS; ++k2) v += red[k2 * 32 * 64 + p];
+        tern_store(a, m, mi, t0 + tl, rbase + col, v);
     }
 }
 

@@ -1,0 +1,451 @@
+// Ternary prefill GEMM on the 6/4-bit matrix instructions: bn_ternary_matmul with T > 32 (model.rs:455-596 qmm_lora /
+// qmm_multi over a prompt; kernels/qmm3.comp).
+//
+// v_mfma_scale_f32_32x32x64_f8f6f4 multiplies fp6 by fp4 at four times the fp16 rate (measured on MI355X: 6.8 against
+// 1.7-1.9 PFLOP/s). Both operands here are exact in those formats:
+//   W: a code c becomes the fp4 value 2 (c - 1) in {-2, 0, 2, 4}; the row's fp16 scale multiplies the sum of each
+//      128-column group in fp32 afterwards (as qmv.glsl:22-35 does), one fma per output and group.
+//   x: 32 columns of a token share the power of two S = 2^floor(log2(max |x|)), and x is written as five fp6 (e2m3)
+//      digits, x = S (n0 + n1 / 32 + ... + n4 / 32^4) / 8 with whole n_i in -16..16 (each the nearest to what the
+//      digits before it left, so exact differences), to within S 2^-24: fp32's own last bit for the block's largest
+//      value. The digit's power of two is the instruction's block scale, so one fp32 accumulator takes all five
+//      (smallest first), and a group's products are summed without a rounding between its columns' scales.
+//   Five MFMAs per 64 columns thus replace the eight of an fp16 hi/lo split, at the same time each.
+// A block of 32 values whose largest is far above the rest (sum |x| < 4 max |x|, and digits that do not end) would
+// leave the small ones with fewer bits than fp32 has: its remainder is written as five more digits and multiplied by
+// a second pass over the group (flagged per 32-token tile; blocks that need none are zero there). The block scale
+// covers fp32's exponents; a block whose sum of |x| is not finite gets the scale NaN, and the token's outputs are NaN.
+// Measured (MI355X, the 4B q/k/v projections of 4,096 tokens): 303 us (digits 17, GEMM 285) against 368 for the fp16
+// hi/lo split, whose 1.16 PFLOP/s of products were the rate of a large library product here; error against 64-bit sums
+// 1.1e-7 of the output's norm against 4.6e-7. The matrix units are busy two thirds of the time at the 1.7 GHz that the
+// power limit leaves (a loop of these MFMAs alone: 1.63 GHz, 157 us for this call's); without the copies the call took
+// 254 us, without the output stores 20 less, and neither another order of the loop nor more stages changed it.
+//
+// Fragment order. MFMA half kh of a group and lane (r = lane % 32, h = lane / 32) hold columns 64 h + 32 kh .. + 31,
+// which are code words 4 h + 2 kh, + 1 of the row: 16 bytes of codes per lane and group. Element e of the 32 is column
+// 16 (e / 8 / 2) + 2 (e % 8) + (e / 8) % 2: a word's even codes, then its odd ones, as the decode leaves them.
+//
+// tern_digits_kernel writes x's digits once per call as the tiles the GEMM reads (15 KB per 32 tokens and group);
+// tern_mx_kernel<W, MT, KS, PRE> multiplies: PRE = true copies those tiles into LDS, false (no workspace) makes the
+// same digits from x itself. Both run the same products in the same order: identical results.
+#pragma once
+#include "bn_ternary.h"
+
+namespace bn {
+
+typedef int i8v __attribute__((ext_vector_type(8)));
+typedef uint32_t u6v __attribute__((ext_vector_type(6)));
+typedef float f32v __attribute__((ext_vector_type(32)));
+
+constexpr int TMX_G = 128;                      // columns per group (one weight scale)
+constexpr int TMX_ND = 5;                       // digits
+constexpr int TMX_FRAG = 64 * 48;               // bytes of a digit: per lane 12 words (kh = 0, then 1) in three 1 KB planes
+constexpr int TMX_DIG = TMX_ND * TMX_FRAG;      // 15,360
+constexpr int TMX_TILE = TMX_DIG + 256;         // a 32-token tile of a group: fragments, then per lane the two scale bytes
+
+// 32-token tiles of a call (an even number: the blocks take two)
+__host__ __device__ inline int tern_mx_tiles(int T) { return 2 * ((T + 63) / 64); }
+// Workspace bytes: per 64 tokens and 64 columns 16 KB and a word (the tiles and flags take 15,620 of the 16,388)
+inline size_t tern_pf_work_bytes(int T, int K) {
+    return (size_t)((T + 63) / 64) * (size_t)(K / 64) * (16384 + 4);
+}
+static_assert(2 * (TMX_TILE + 4) <= 2 * (16384 + 4), "the workspace holds the tiles and their flags");
+
+// The digits of 32 values of a token. In: x by element (u[i] = element 2 i, v[i] = element 2 i + 1). Out: each
+// digit's six words through put(d, words), the remainders in u and v, whether they need a second set of digits in wide;
+// returns the block's scale byte.
+struct TernBlock {
+    f16x u, v;
+};
+__device__ __forceinline__ float tern_pow2(int e) { return __int_as_float(e << 23); }
+template <typename Put>
+__device__ __forceinline__ int tern_digits(TernBlock& x, bool& wide, const Put& put) {
+    float mx = 0.0f, sum = 0.0f;  // an infinity or a NaN shows in the sum (as do finite values whose sum overflows)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(mx) : "v"(x.u[i]), "v"(x.v[i]));
+        sum += fabsf(x.u[i]) + fabsf(x.v[i]);
+    }
+    const int e = sum < INFINITY ? max(__float_as_int(mx) >> 23, 28) : 255;  // 28: the last digit's scale stays normal
+    const bool spread = sum < 4.0f * mx;  // the largest value far above the rest
+#pragma unroll
+    for (int d = 0; d < TMX_ND; ++d) {
+        const float sc = tern_pow2(e - 5 * d);
+        const u6v q = __builtin_bit_cast(u6v, __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(x.u, x.v, sc));
+        put(d, q);
+        if (d == TMX_ND - 1 && __ballot(spread) == 0) break;
+        const f32v b = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(q, sc);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            x.u[i] -= b[2 * i];
+            x.v[i] -= b[2 * i + 1];
+        }
+    }
+    wide = false;
+    if (spread) {
+        uint32_t rest = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) rest |= __float_as_uint(x.u[i]) | __float_as_uint(x.v[i]);
+        wide = (rest & 0x7FFFFFFFu) != 0;
+    }
+    return e;
+}
+// element e of the fragment order: its column in the 32
+__host__ __device__ constexpr int tern_mx_col(int e) { return 16 * (e >> 4) + 2 * (e & 7) + ((e >> 3) & 1); }
+// 32 floats, 16 bytes at a time through ld(i) (floats 4 i .. 4 i + 3), in element order
+template <typename Ld>
+__device__ __forceinline__ void tern_block_load(TernBlock& x, const Ld& ld) {
+    f4 c[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) c[i] = ld(i);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int a = tern_mx_col(2 * i), b = tern_mx_col(2 * i + 1);
+        x.u[i] = c[a >> 2][a & 3];
+        x.v[i] = c[b >> 2][b & 3];
+    }
+}
+// digit d's six words of (lane, kh) into a tile at p (global memory or LDS): words 6 kh .. of the lane's 12, four of
+// them in each 1 KB plane, so that a lane reads both halves' operands in three 16-byte reads
+__device__ __forceinline__ void tern_mx_put(uint8_t* p, int kh, int d, int lane, u6v q) {
+    uint8_t* f = p + d * TMX_FRAG + 16 * lane;
+    *reinterpret_cast<u4*>(f + (kh ? 2048 : 0)) = kh ? u4{q[2], q[3], q[4], q[5]} : u4{q[0], q[1], q[2], q[3]};
+    *reinterpret_cast<u2*>(f + 1024 + 8 * kh) = kh ? u2{q[0], q[1]} : u2{q[4], q[5]};
+}
+
+typedef __attribute__((address_space(3))) void tmx_lds_t;
+// 16 (4) bytes per lane from global memory into LDS at lds + 16 lane (4 lane)
+__device__ __forceinline__ void tmx_copy16(const void* g, const uint8_t* lds) {
+    __builtin_amdgcn_global_load_lds(g, (tmx_lds_t*)const_cast<uint8_t*>(lds), 16, 0, 0);
+}
+__device__ __forceinline__ void tmx_copy4(const void* g, const uint8_t* lds) {
+    __builtin_amdgcn_global_load_lds(g, (tmx_lds_t*)const_cast<uint8_t*>(lds), 4, 0, 0);
+}
+
+// x's digits: one block per 64 tokens and group; work: [tile][group] TMX_TILE bytes, then a flag word each. The rows
+// come through LDS (a copy moves 512 contiguous bytes of two tokens; a thread then takes 32 columns of one token):
+// read straight into registers, a wave would touch 64 lines per load. Tokens past T get zeros.
+__global__ __launch_bounds__(256) void tern_digits_kernel(const float* __restrict__ x, int64_t x_ts, int T, int K,
+                                                          uint8_t* __restrict__ work) {
+    constexpr int PAIR = 1040;  // LDS pitch of two tokens' 512 bytes
+    __shared__ __attribute__((aligned(16))) uint8_t rows[32 * PAIR];
+    const int ng = K / TMX_G;
+    const int tt = (int)blockIdx.x / ng, g = (int)blockIdx.x - tt * ng, t0 = 64 * tt;
+    const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        // an odd token's 16-byte chunks are swapped in blocks of 8, so that 16 tokens' reads fall on distinct banks
+        const int p = 8 * wave + i, odd = lane >> 5, t = min(t0 + 2 * p + odd, T - 1);
+        tmx_copy16(x + (int64_t)t * x_ts + g * TMX_G + 4 * ((lane & 31) ^ (8 * odd)), rows + p * PAIR);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    // wave: tile wave / 2, lane half h = wave % 2 of its fragments; lane: token lane % 32, half kh = lane / 32
+    const int u = wave >> 1, h = wave & 1, m = lane & 31, kh = lane >> 5, b = 2 * h + kh;
+    const int tile = 2 * tt + u;
+    uint8_t* out = work + ((size_t)tile * ng + g) * TMX_TILE;
+    TernBlock v;
+    const uint8_t* src = rows + (16 * u + (m >> 1)) * PAIR + 512 * (m & 1);
+    tern_block_load(v, [&](int i) { return *reinterpret_cast<const f4*>(src + 16 * ((8 * b + i) ^ (8 * (m & 1)))); });
+    if (t0 + 32 * u + m >= T) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v.u[i] = v.v[i] = 0.0f;
+    }
+    bool wide;
+    const int e = tern_digits(v, wide, [&](int d, u6v q) { tern_mx_put(out, kh, d, m + 32 * h, q); });
+    out[TMX_DIG + 4 * (m + 32 * h) + kh] = (uint8_t)e;
+    __shared__ int wide_lds[4];
+    const bool any = __ballot(wide) != 0;
+    if (lane == 0) wide_lds[wave] = any;
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        uint32_t* flags = reinterpret_cast<uint32_t*>(work + (size_t)tern_mx_tiles(T) * ng * TMX_TILE);
+        flags[(size_t)(2 * tt + threadIdx.x) * ng + g] = wide_lds[2 * threadIdx.x] | wide_lds[2 * threadIdx.x + 1];
+    }
+}
+
+// 32 codes (two words) as fp4 values 2 (c - 1): bit 3 = !b1, bit 2 = !b0 | b1, bit 1 = b0 & b1 of the code's bits;
+// words 0, 1: the even and the odd codes of w0, 2, 3: of w1
+__device__ __forceinline__ void tern_fp4(uint32_t w, int& even, int& odd) {
+    const uint32_t v = w >> 1, n = ~w | (v & 0x55555555u);
+    uint32_t q = w & v & 0x55555555u;
+    asm("" : "+v"(q));  // the selects below stay v_bfi_b32 (knowing q's zero bits, the compiler masks and ors instead)
+    even = (int)(((n << 2) & 0xCCCCCCCCu) | ((q << 1) & ~0xCCCCCCCCu));
+    odd = (int)((n & 0xCCCCCCCCu) | ((q >> 1) & ~0xCCCCCCCCu));
+}
+
+// stage bytes of a wave group: its MT x tiles, then the waves' codes (64 rows x 32 bytes each)
+__host__ __device__ constexpr int tmx_stage(int W, int MT) { return MT * TMX_TILE + W * 2048; }
+// copies of fragments per wave and group of columns (1 KB each, the last repeated where they do not divide)
+__host__ __device__ constexpr int tmx_frag_copies(int W, int MT) { return (15 * MT + W - 1) / W; }
+
+// KS wave groups of W waves x 64 rows, 32 MT tokens; the groups split the columns and add their sums at the end, in
+// order. PRE: x's digits come from tern_digits_kernel's tiles, otherwise from x. Per 128 columns a wave multiplies MT
+// token tiles x 2 row tiles x 2 halves x 5 digits (32 cycles each) into a fresh accumulator per tile pair, which one
+// fma per output adds, times the row scale, to the running sums. Two stages in LDS, the next step's copies in flight
+// during a step's products; one barrier per step.
+template <int W, int MT, int KS, bool PRE>
+__global__ __launch_bounds__(64 * W * KS, 2) void tern_mx_kernel(TernArgs a, int row_tiles,
+                                                                 const uint8_t* __restrict__ work) {
+    static_assert(MT == 1 || MT == 2, "token tiles per block (x's tiles come in pairs)");
+    constexpr int BM = 32 * MT, STAGE = tmx_stage(W, MT), ST_W = MT * TMX_TILE;
+    // separate arrays, so that the compiler can tell one stage's copies from another's reads
+    __shared__ __attribute__((aligned(1024))) uint8_t lds0[KS * STAGE];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds1[KS * STAGE];
+    __shared__ int wide_lds[2][W * KS];
+    static_assert(KS == 1 || (KS - 1) * W * MT * 8192 <= KS * STAGE, "the groups' sums fit a stage");
+    const int lane = (int)threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), ks = wv / W, wave = wv % W;
+    const int n = lane & 31, h = lane >> 5;
+    int rt, tt;
+    tern_tile<BM, (BN_TERN_XCD_GROUP * 64 / BM > 0 ? BN_TERN_XCD_GROUP * 64 / BM : 1)>((int)blockIdx.x, row_tiles, a.T, rt, tt);
+    const int t0 = tt * BM;
+    const int rbase_g = (rt * W + wave) * 64;  // first global row of this wave
+    const bool active = rbase_g < a.rows;
+    int rbase = active ? rbase_g : 0;          // inactive waves take member 0's first rows (in bounds, not stored)
+    const int mi = tern_member(a, rbase);
+    const TernMat m = tern_mat(a, mi);
+    const int K = a.K, kw = K >> 4, ng = K / TMX_G;
+    // the wave group's 128-column groups [g0, g0 + cnt); a step past cnt repeats a group's copies, unused
+    const int g0 = ks * ng / KS, cnt = (ks + 1) * ng / KS - g0, steps = (ng + KS - 1) / KS;
+    int cnt_ = cnt;
+    asm("" : "+s"(cnt_));
+    auto group = [&](int j) { return min(g0 + min(j, cnt - 1 > 0 ? cnt - 1 : 0), ng - 1); };
+    const int ntiles = tern_mx_tiles(a.T);
+    const size_t xt = (size_t)MT * tt;  // the block's first x tile
+    const size_t tile_row = (size_t)ng * TMX_TILE;
+    const uint8_t* tiles = work + xt * tile_row;
+    const uint32_t* flags = reinterpret_cast<const uint32_t*>(work + ntiles * tile_row) + xt * ng;
+    // A copy of row tile nt's codes takes a row's two 16-byte halves with neighbouring lanes (a load of 64 separate
+    // places costs the address unit 64 cycles, and these loads bound small calls): lane -> row lane / 2, half
+    // lane % 2, the halves swapped in every other 8 rows so that the operand reads fall on distinct banks
+    const int cr = lane >> 1, ch = (lane & 1) ^ ((cr >> 3) & 1);
+    const uint8_t* wsrc = reinterpret_cast<const uint8_t*>(m.w + (int64_t)(rbase + cr) * kw) + 16 * ch;
+    const int64_t wtile = (int64_t)32 * kw * 4;
+    const int w_lane = wave * 2048 + 32 * n + 16 * (h ^ ((n >> 3) & 1));
+    // scales of rows n, 32 + n: four groups' at a time where they lie on 8 bytes (for the same reason), else one
+    const bool s4 = (ng & 3) == 0 && ((uintptr_t)m.s & 7) == 0;
+    const uint16_t* ssrc = m.s + (int64_t)(rbase + n) * ng;
+    uint64_t sw[2];
+    auto load_s = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+            const uint16_t* p = ssrc + (int64_t)32 * nt * ng + g;
+            if (s4)
+                sw[nt] = *reinterpret_cast<const uint64_t*>(p - (g & 3));
+            else
+                sw[nt] = *p;
+        }
+    };
+    // the copies of column group g into a stage
+    auto issue = [&](int g, const uint8_t* sb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) tmx_copy16(wsrc + nt * wtile + 32 * g, sb + ST_W + wave * 2048 + nt * 1024);
+        if constexpr (PRE) {
+            constexpr int C = tmx_frag_copies(W, MT);
+#pragma unroll
+            for (int i = 0; i < C; ++i) {
+                const int f = min(wave * C + i, 15 * MT - 1), u = f / 15, o = (f - 15 * u) * 1024;
+                tmx_copy16(tiles + u * tile_row + (size_t)g * TMX_TILE + o + 16 * lane, sb + u * TMX_TILE + o);
+            }
+            const int u = wave & (MT - 1);
+            tmx_copy4(tiles + u * tile_row + (size_t)g * TMX_TILE + TMX_DIG + 4 * lane, sb + u * TMX_TILE + TMX_DIG);
+        }
+    };
+    // x itself, for PRE = false and the second passes. Thread u of the wave group -> tile, token, 32 columns.
+    const int u_ = (int)threadIdx.x - 64 * W * ks;
+    const int xtile = u_ >> 7, xh = (u_ >> 6) & 1, xkh = (u_ >> 5) & 1, xm = u_ & 31, xtok = t0 + 32 * xtile + xm;
+    auto load_x = [&](int g, TernBlock& v) __attribute__((always_inline)) {
+        const float* p = a.x + (int64_t)min(xtok, a.T - 1) * a.x_ts + g * TMX_G + 64 * xh + 32 * xkh;
+        tern_block_load(v, [&](int c) { return reinterpret_cast<const f4*>(p)[c]; });
+    };
+    // the thread's 32 values as digits into a stage (second: their remainders' digits where they need them, else zeros);
+    // returns whether they need a second set
+    auto make_tiles = [&](TernBlock& v, uint8_t* sb, bool second) __attribute__((always_inline)) {
+        if (xtile >= MT) return false;
+        uint8_t* dst = sb + xtile * TMX_TILE;
+        bool wide = false, drop = xtok >= a.T;
+        int e = 0;
+#pragma unroll 1
+        for (int pass = second ? 0 : 1; pass < 2; ++pass) {
+            if (drop) {
+#pragma unroll
+                for (int c = 0; c < 16; ++c) v.u[c] = v.v[c] = 0.0f;
+            }
+            e = tern_digits(v, wide, [&](int d, u6v q) { tern_mx_put(dst, xkh, d, xm + 32 * xh, q); });
+            drop = !wide;
+        }
+        dst[TMX_DIG + 4 * (xm + 32 * xh) + xkh] = (uint8_t)e;
+        return wide;
+    };
+    static_assert(128 * MT <= 64 * W, "a thread per 32 columns of a token");
+
+    f16x acc[MT][2];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][nt][e] = 0.0f;
+
+    // the digits' powers of two, 2^(-5 d) / 2: fp4 weights are twice c - 1
+    const int sw0 = 126 | (121 << 8) | (116 << 16) | (111 << 24), sw1 = 106;
+    // the products of a group: codes decoded, then per token tile five digits x two halves, smallest digit first
+    auto products = [&](const uint8_t* sb, const float (&sc)[2]) __attribute__((always_inline)) {
+        i8v b[2][2];
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+            const u4 wc = *reinterpret_cast<const u4*>(sb + ST_W + w_lane + nt * 1024);
+#pragma unroll
+            for (int kh = 0; kh < 2; ++kh) {
+                int w0, w1, w2, w3;
+                tern_fp4(wc[2 * kh], w0, w1);
+                tern_fp4(wc[2 * kh + 1], w2, w3);
+                b[nt][kh] = i8v{w0, w1, w2, w3, 0, 0, 0, 0};
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            const uint8_t* xl = sb + i * TMX_TILE;
+            const int ex = *reinterpret_cast<const int*>(xl + TMX_DIG + 4 * lane);
+            f16x t[2];
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) t[nt][e] = 0.0f;
+#pragma unroll
+            for (int d = TMX_ND - 1; d >= 0; --d) {
+                const u4* f = reinterpret_cast<const u4*>(xl + d * TMX_FRAG + 16 * lane);
+                const u4 w0 = f[0], w1 = f[64], w2 = f[128];
+                const i8v x0 = {(int)w0[0], (int)w0[1], (int)w0[2], (int)w0[3], (int)w1[0], (int)w1[1], 0, 0};
+                const i8v x1 = {(int)w1[2], (int)w1[3], (int)w2[0], (int)w2[1], (int)w2[2], (int)w2[3], 0, 0};
+                // the scale operands' byte selects are immediates: one call per digit
+#define TMX_MFMA(DD, SW)                                                                                        \
+    for (int nt = 0; nt < 2; ++nt)                                                                              \
+        t[nt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x0, b[nt][0], t[nt], 2, 4, 0, ex, DD, SW);      \
+    for (int nt = 0; nt < 2; ++nt)                                                                              \
+        t[nt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x1, b[nt][1], t[nt], 2, 4, 1, ex, DD, SW)
+                if (d == 4) { TMX_MFMA(0, sw1); }
+                if (d == 3) { TMX_MFMA(3, sw0); }
+                if (d == 2) { TMX_MFMA(2, sw0); }
+                if (d == 1) { TMX_MFMA(1, sw0); }
+                if (d == 0) { TMX_MFMA(0, sw0); }
+#undef TMX_MFMA
+            }
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[i][nt][e] = fmaf(t[nt][e], sc[nt], acc[i][nt][e]);
+        }
+    };
+
+    // whether some group of the block's tiles needs a second pass, read before the copies
+    bool block_wide = false;
+    if constexpr (PRE) {
+        uint32_t f = 0;
+        for (int g = lane; g < ng; g += 64)
+#pragma unroll
+            for (int u = 0; u < MT; ++u) f |= flags[(size_t)u * ng + g];
+        block_wide = __ballot(f != 0) != 0;
+    }
+    auto stage_tiles = [&](TernBlock& v, uint8_t* sb, int s) __attribute__((always_inline)) {
+        const bool any = __ballot(make_tiles(v, sb, false)) != 0;
+        if (lane == 0) wide_lds[s][wv] = any;
+    };
+    uint8_t* const st0 = lds0 + ks * STAGE;
+    uint8_t* const st1 = lds1 + ks * STAGE;
+    load_s(group(0));
+    issue(group(0), st0);
+    if constexpr (!PRE) {
+        TernBlock v;
+        load_x(group(0), v);
+        stage_tiles(v, st0, 0);
+    }
+
+    // step j from stage sb (s: its number) while step j + 1 is brought into nb
+    auto step = [&](int j, uint8_t* sb, uint8_t* nb, int s) __attribute__((always_inline)) {
+        // this step's copies of every wave have landed, and every wave is done with nb
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        const int g = group(j), gn = group(j + 1);
+        float sc[2];
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+            asm volatile("" : "+v"(sw[nt]));  // the compiler's wait for this load ends here, before the next copies
+            sc[nt] = h2f((uint16_t)(sw[nt] >> (s4 ? 16 * (g & 3) : 0)));
+        }
+        if (!s4 || (gn & 3) == 0) load_s(gn);
+        bool wide = false;  // the same for every wave of the block
+        if constexpr (PRE) {
+            if (block_wide) {
+#pragma unroll
+                for (int q = 0; q < KS; ++q) {
+                    const int q0 = q * ng / KS, gq = min(q0 + j, max((q + 1) * ng / KS - 1, 0));
+#pragma unroll
+                    for (int u = 0; u < MT; ++u) wide |= flags[(size_t)u * ng + gq] != 0;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int w = 0; w < W * KS; ++w) wide |= wide_lds[s][w] != 0;
+        }
+        issue(gn, nb);
+        TernBlock v;  // PRE = false: the next step's x, in flight during the products
+        if constexpr (!PRE) load_x(gn, v);
+        // PRE = false always branches here (in one piece with the digits below, the compiler spills registers)
+        if ((KS == 1 && PRE) || j < cnt_) products(sb, sc);
+        if constexpr (!PRE) {
+            stage_tiles(v, nb, s ^ 1);
+        }
+        if (wide) {
+            // rare: the remainders of the blocks that need them take the tiles' place
+            __syncthreads();
+            load_x(g, v);
+            make_tiles(v, sb, true);
+            __syncthreads();
+            if (KS == 1 || j < cnt) products(sb, sc);
+        }
+    };
+    for (int j = 0; j < steps; j += 2) {
+        step(j, st0, st1, 0);
+        if (j + 1 < steps) step(j + 1, st1, st0, 1);
+    }
+    // the last copies (repeats into free stages) land before the block's LDS is reused or released
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+    if constexpr (KS > 1) {
+        // the groups' sums, added in group order by the first group's waves
+        float* red = reinterpret_cast<float*>(lds0);
+        __syncthreads();
+        auto slot = [&](int q, int i, int nt, int e) { return ((((q * W + wave) * MT + i) * 2 + nt) * 16 + e) * 64 + lane; };
+        if (ks > 0)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) red[slot(ks - 1, i, nt, e)] = acc[i][nt][e];
+        __syncthreads();
+        if (ks > 0) return;
+#pragma unroll
+        for (int q = 0; q < KS - 1; ++q)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[i][nt][e] += red[slot(q, i, nt, e)];
+    }
+    // C layout: acc[i][nt][j] = (token 32 i + 8 (j / 4) + 4 h + j % 4, row 32 nt + n)
+    if (!active) return;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int t = t0 + 32 * i + 8 * (j >> 2) + 4 * h + (j & 3);
+            if (t < a.T)
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt) tern_store(a, m, mi, t, rbase + 32 * nt + n, acc[i][nt][j]);
+        }
+}
+
+}  // namespace bn

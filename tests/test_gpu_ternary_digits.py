@@ -1,0 +1,86 @@
+"""bn_ternary_matmul with more than 32 tokens (bn_ternary_mx.h) against float64: x as five base-32 digits per block of 32
+columns of a token, with a second set where one value of a block is far above the rest.
+
+Bound per output, from the arithmetic: a block's digits end within 2^-24 of the power of two below its largest value
+(for a block with a second set: of its remainder's, so 2^-44), and each group's sum takes at most 20 additions of MFMA
+results and one fma, each rounding the running sum by at most 2^-23 of sum |x w| (2^-24 for one rounding, doubled for an
+accumulation inside the MFMA); the groups' sums add one more each.
+"""
+import numpy as np
+import pytest
+
+import oracle
+import workload
+from glimpse_language_amd import bonsai_attn as ba
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(torch, a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def call(torch, ctx, mats, x, work):
+    xd = dev(torch, x)
+    ys = [torch.full((x.shape[0], w.shape[0]), float("nan"), device="cuda") for w, _, _ in mats]
+    ws = ba.ternary_workspace(xd) if work else None
+    if work:
+        ws.fill_(0xA5)
+    ba.ternary_matmul(ctx, xd, [(dev(torch, w.view(np.int32)), dev(torch, s.view(np.int16)), y)
+                                for (w, s, _), y in zip(mats, ys)], work=ws)
+    torch.cuda.synchronize()
+    return [y.cpu().numpy() for y in ys]
+
+
+def exact(w, s, codes, x):
+    full = (codes.astype(np.float64) - 1) * np.repeat(oracle.f16_to_f32(s).astype(np.float64), 128, axis=1)
+    x = x.astype(np.float64)
+    blocks = np.abs(x).reshape(x.shape[0], -1, 32)
+    mx = blocks.max(-1)
+    cut = np.where(blocks.sum(-1) < 4 * mx, 2.0 ** -44, 2.0 ** -24) * mx
+    aw = np.abs(full)
+    split = cut @ aw.reshape(aw.shape[0], -1, 32).sum(-1).T
+    groups = x.shape[1] // 128
+    return x @ full.T, split + (21 + groups) * 2.0 ** -23 * (np.abs(x) @ aw.T)
+
+
+# tokens at the edges of the 32- and 64-token tiles; one group (the second wave group has it alone), three (odd, scales
+# one at a time), rows that leave 128- and 256-row blocks partly empty; 32 x 256 blocks; 64 x 256 blocks
+SHAPES = [(33, 128, (64,)), (64, 384, (192,)), (65, 512, (320, 64)), (97, 2048, (128,)), (500, 256, (4096, 512, 512)),
+          (1025, 256, (4096, 512, 512))]
+
+
+@pytest.mark.parametrize("T,K,os", SHAPES)
+def test_digits_against_float64(gpu, T, K, os):
+    torch, ctx, _ = gpu
+    print(f"ternary digits T={T} K={K} os={os}", flush=True)
+    mats = [workload.ternary_weights(0x7A00 + T + i, o, K, True) for i, o in enumerate(os)]
+    x = oracle.normal(0x7A00 + T, 1, (T, K)).copy()
+    # blocks that need a second set (in the first, a middle and the last token), a block of one value and zeros, tiny
+    # values, values whose digits end early
+    x[0, 5], x[T // 2, K - 1], x[T - 1, 40] = 3.0e4, -1.0e7, 700.0
+    x[1, :32] = 0.0
+    x[1, 3] = 1.1
+    x[2] *= 2.0 ** -60
+    x[3] = np.round(x[3] * 4)
+    got = call(torch, ctx, mats, x, True)
+    for g, (w, s, codes) in zip(got, mats):
+        ref, tol = exact(w, s, codes, x)
+        bad = np.argwhere(~(np.abs(g - ref) <= tol))
+        assert bad.size == 0, f"{len(bad)} outputs off, first {bad[:3].tolist()}"
+    assert all(np.array_equal(a, b) for a, b in zip(got, call(torch, ctx, mats, x, False))), "without a workspace"
+
+
+def test_digits_nonfinite_token(gpu):
+    """An infinity or a NaN makes its own token's outputs NaN and leaves the others as they are."""
+    torch, ctx, _ = gpu
+    T, K, os = 70, 384, (128,)
+    mats = [workload.ternary_weights(0x7B00, os[0], K, False)]
+    x = oracle.normal(0x7B00, 1, (T, K)).copy()
+    clean = call(torch, ctx, mats, x, True)[0]
+    x[4, 200], x[66, 0] = np.inf, np.nan
+    for work in (True, False):
+        got = call(torch, ctx, mats, x, work)[0]
+        assert np.isnan(got[[4, 66]]).all()
+        rest = np.setdiff1d(np.arange(T), [4, 66])
+        assert np.array_equal(got[rest], clean[rest])
