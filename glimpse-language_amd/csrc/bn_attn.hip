@@ -13,7 +13,6 @@
 #include <utility>
 
 #include "bn_decode.h"
-#include "bn_flash.h"
 #include "bn_prefill.h"
 #include "bn_prefill_hilo.h"
 #include "bn_prefill_pair.h"
@@ -36,13 +35,13 @@ struct bn_ctx {
     int decode_target_waves;
     // splits of one sequence at most (1 .. kMaxSplitsCap; BONSAI_ATTN_DECODE_MAX_SPLITS)
     int decode_max_splits;
-    // blocks flash_kernel's key splits aim at (1 .. kFlashTargetBlocks; BONSAI_ATTN_FLASH_TARGET_BLOCKS)
-    int flash_target_blocks;
+    // blocks that split key ranges may give (1 .. kSplitTarget; BONSAI_ATTN_FLASH_TARGET_BLOCKS)
+    int split_target_blocks;
     // 2..16 verify rows on verify_kernel (1, the default) or as decodes of their rows (0; BONSAI_ATTN_VERIFY_MFMA)
     int verify_mfma;
     // fp16-q prefills on prefill_kernel (0, the default) or prefill_pair_kernel (1; BONSAI_ATTN_PREFILL_PAIR=1)
     int prefill_pair;
-    // 17..64 rows too few for prefill_kernel: verify_kernel's row groups (1, the default) or flash_kernel (0;
+    // 17..64 rows too few for prefill_kernel: verify_kernel's row groups (1, the default) or q-tiles with split keys (0;
     // BONSAI_ATTN_MID_ROWS)
     int mid_rows;
     // this device's copy of `scratch` (the partials of bn_attn_decode_ragged_noalloc), or null if its address
@@ -175,40 +174,58 @@ DecodePlan plan_rows(const bn_attn_args* a, int64_t waves, int64_t target_waves,
     return p;
 }
 
-// T >= 2 rows: q-tiles of 32 tokens; the key range of a q-tile is split only when the q-tiles alone give
-// fewer blocks than CUs (then about 512 blocks of equal key tiles). Depends only on the shapes.
-// flash_kernel's key splits aim at about this many blocks (the workspace query sizes the partials for it; a context
-// may aim lower: BONSAI_ATTN_FLASH_TARGET_BLOCKS)
-constexpr int64_t kFlashTargetBlocks = 512;
+// T >= 2 rows: q-tiles of 32 tokens of the 4 query heads of a kv head, one block each (prefill_hilo_kernel: one block per
+// CU, so kSplitTarget blocks run at once). When the q-tiles alone leave CUs idle, each q-tile's key tiles are cut into
+// ceil(nt / ct) equal splits, ct the least number that gives no more blocks than that: a block costs a start (q rows,
+// the first tiles, about 4 us) and a 128 KB record besides about 2 us per key tile, so a second round of blocks loses
+// more than it balances (777 rows over 1,031, 16/4 heads: 44 us a call in one round, 60 with the XCDs' shares uneven).
+// At least 3 tiles a split, or 2 where that gives no more than half the blocks (256 rows over 512, 8/2 heads: 25.1
+// with 3, 26.0 with 4, 27.9 with 6; a layer call of 70 rows over none: 23.7 with 2, 28.2 unsplit). Depends only on the
+// shapes.
+constexpr int64_t kSplitTarget = 256;
 
-struct FlashPlan {
-    int64_t ntq, ct, max_splits;
+struct SplitPlan {
+    int64_t ntq, ct, max_splits, blocks;
     size_t acc_bytes, ml_bytes;
     size_t total() const { return max_splits > 1 ? acc_bytes + ml_bytes : 0; }
 };
 
-FlashPlan plan_flash(int64_t T, int64_t off, int64_t KV, int64_t target_blocks = kFlashTargetBlocks) {
-    FlashPlan p;
-    p.ntq = ceil_div(T, bn::FL_BQ);
-    const int64_t max_kt = ceil_div(off + T, bn::FL_BK);
-    if (KV * p.ntq >= 256) {
-        p.ct = max_kt;
-    } else {
-        int64_t iters = 0;
-        for (int64_t qt = 0; qt < p.ntq; qt++) {
-            const int64_t t_last = (qt + 1) * bn::FL_BQ < T ? (qt + 1) * bn::FL_BQ : T;
-            iters += ceil_div(off + t_last, bn::FL_BK);
+SplitPlan plan_split(int64_t T, int64_t off, int64_t KV, int64_t target_blocks = kSplitTarget) {
+    SplitPlan p;
+    p.ntq = ceil_div(T, bn::PF_BQ);
+    auto tiles = [&](int64_t qt) {  // key tiles of a q-tile
+        const int64_t t_end = (qt + 1) * bn::PF_BQ < T ? (qt + 1) * bn::PF_BQ : T;
+        return ceil_div(off + t_end, bn::PF_BK);
+    };
+    const int64_t max_nt = tiles(p.ntq - 1);
+    p.ct = max_nt;
+    p.blocks = KV * p.ntq;
+    if (KV * p.ntq < target_blocks) {
+        auto blocks = [&](int64_t ct) {
+            int64_t n = 0;
+            for (int64_t qt = 0; qt < p.ntq; qt++) n += ceil_div(tiles(qt), ct);
+            return n * KV;
+        };
+        int64_t lo = 2 * blocks(2) <= target_blocks ? 2 : 3, hi = max_nt;
+        if (lo > max_nt) lo = max_nt;
+        while (lo < hi) {  // the number of blocks falls with ct: bisection
+            const int64_t mid = (lo + hi) / 2;
+            if (blocks(mid) <= target_blocks) hi = mid;
+            else lo = mid + 1;
         }
-        iters *= KV;
-        p.ct = ceil_div(iters, target_blocks);
-        if (p.ct < 1) p.ct = 1;
+        p.ct = lo;
+        p.blocks = blocks(lo);
     }
-    p.max_splits = ceil_div(max_kt, p.ct);
-    const int64_t rows = KV * p.ntq * p.max_splits * bn::FL_ROWS;
+    p.max_splits = ceil_div(max_nt, p.ct);
+    const int64_t rows = KV * p.ntq * p.max_splits * bn::PF_ROWS;
     p.acc_bytes = (size_t)rows * bn::D * sizeof(float);
     p.ml_bytes = (size_t)rows * 2 * sizeof(float);
     return p;
 }
+
+// key tiles in which such a call's running max is exact: a short range (or split) keeps the precision of 64-key splits
+// with the max taken over each (simulated and measured: 1.6e-4 of the output at 128 keys, 1.9e-4 without)
+constexpr int kSplitExact = 5;
 
 // T >= 2 rows with enough 32-token q-tiles to fill the GPU: prefill_kernel (one block per q-tile, the key range
 // split between the block's two wave groups). Depends only on the shapes and the context's threshold.
@@ -558,7 +575,8 @@ bn_status run_verify(bn_ctx* ctx, hipStream_t st, const bn_attn_args* a, int64_t
     return launched(ctx, "decode_combine_kernel");
 }
 
-bn_status run_prefill(bn_ctx* ctx, hipStream_t st, const bn_attn_args* a) {
+// q-tiles of T >= 2 rows, whole (split null or one split) or with their key ranges split; the kernels gate and rotate.
+bn_status run_prefill(bn_ctx* ctx, hipStream_t st, const bn_attn_args* a, const SplitPlan* split) {
     bn::PrefillArgs f{};
     if (a->flags & BN_Q_F16)
         f.q16 = static_cast<const uint16_t*>(a->q);
@@ -580,7 +598,30 @@ bn_status run_prefill(bn_ctx* ctx, hipStream_t st, const bn_attn_args* a) {
     f.off = (int)a->off;
     f.KV = (int)a->KV;
     f.ntq = (int)ceil_div(a->T, bn::PF_BQ);
-    const int64_t blocks = (int64_t)a->KV * f.ntq;
+    int64_t blocks = (int64_t)a->KV * f.ntq;
+    f.exact = split ? kSplitExact : 1;
+    if (split && split->max_splits > 1) {
+        f.part_acc = static_cast<float*>(a->ws);
+        f.part_ml = reinterpret_cast<float*>(static_cast<char*>(a->ws) + split->acc_bytes);
+        f.ct = (int)split->ct;
+        f.max_splits = (int)split->max_splits;
+        blocks = split->blocks;
+        if (f.q16)
+            bn_launch(ctx, (bn::prefill_hilo_kernel<false, true>), dim3((unsigned)blocks), dim3(256), 0, st, f);
+        else
+            bn_launch(ctx, (bn::prefill_hilo_kernel<true, true>), dim3((unsigned)blocks), dim3(256), 0, st, f);
+        bn_status s = launched(ctx, "prefill_hilo_kernel (split)");
+        if (s) return s;
+        bn_launch(ctx, bn::prefill_combine_kernel, dim3(a->T, 2 * a->KV), dim3(64), 0, st, f);
+        return launched(ctx, "prefill_combine_kernel");
+    }
+    if (split) {
+        if (f.q16)
+            bn_launch(ctx, (bn::prefill_hilo_kernel<false, false>), dim3((unsigned)blocks), dim3(256), 0, st, f);
+        else
+            bn_launch(ctx, (bn::prefill_hilo_kernel<true, false>), dim3((unsigned)blocks), dim3(256), 0, st, f);
+        return launched(ctx, "prefill_hilo_kernel");
+    }
     if (f.q16 && ctx->prefill_pair) {
         bn_launch(ctx, bn::prefill_pair_kernel, dim3((unsigned)blocks), dim3(256), 0, st, f);
         return launched(ctx, "prefill_pair_kernel");
@@ -589,80 +630,17 @@ bn_status run_prefill(bn_ctx* ctx, hipStream_t st, const bn_attn_args* a) {
         bn_launch(ctx, bn::prefill_kernel, dim3((unsigned)blocks), dim3(512), 0, st, f);
         return launched(ctx, "prefill_kernel");
     }
-    bn_launch(ctx, bn::prefill_hilo_kernel, dim3((unsigned)blocks), dim3(256), 0, st, f);
+    bn_launch(ctx, (bn::prefill_hilo_kernel<true, false>), dim3((unsigned)blocks), dim3(256), 0, st, f);
     return launched(ctx, "prefill_hilo_kernel");
 }
 
-// T >= 2 rows: append, then the MFMA kernel (and the split merge when the key range is split).
-bn_status attend_flash(bn_ctx* ctx, hipStream_t st, const bn_attn_args* a) {
-    if (a->k_new) {
-        bn_status s = launch_append(ctx, st, a);
-        if (s) return s;
-    }
-    if (use_prefill(a, ctx->prefill_min_blocks)) return run_prefill(ctx, st, a);
-    FlashPlan p = plan_flash(a->T, a->off, a->KV, ctx->flash_target_blocks);
-    bn::FlashArgs f{};
-    if (a->flags & BN_Q_F16)
-        f.q16 = static_cast<const uint16_t*>(a->q);
-    else
-        f.q = static_cast<const float*>(a->q);
-    f.q_ts = a->q_ts;
-    f.q_hs = a->q_hs;
-    f.kc = a->kc;
-    f.vc = a->vc;
-    f.gate = a->gate;
-    f.g_ts = a->g_ts;
-    f.g_hs = a->g_hs;
-    f.out = a->out;
-    f.o_ts = a->o_ts;
-    f.o_hs = a->o_hs;
-    f.T = (int)a->T;
-    f.off = (int)a->off;
-    f.KV = (int)a->KV;
-    f.ntq = (int)p.ntq;
-    f.ct = (int)p.ct;
-    f.max_splits = (int)p.max_splits;
-    f.dyn = a->dyn;
-    if (p.max_splits > 1) {
-        f.part_acc = static_cast<float*>(a->ws);
-        f.part_ml = reinterpret_cast<float*>(static_cast<char*>(a->ws) + p.acc_bytes);
-    }
-    const int64_t blocks = (int64_t)a->KV * p.ntq * p.max_splits;
-    if (f.q16)
-        bn_launch(ctx, (bn::flash_kernel<false>), dim3((unsigned)blocks), dim3(256), 0, st, f);
-    else
-        bn_launch(ctx, (bn::flash_kernel<true>), dim3((unsigned)blocks), dim3(256), 0, st, f);
-    bn_status s = launched(ctx, "flash_kernel");
-    if (s || p.max_splits == 1) return s;
-    bn_launch(ctx, bn::flash_combine_kernel, dim3(a->T, a->H), dim3(64), 0, st, f);
-    return launched(ctx, "flash_combine_kernel");
-}
-
-// The rotation of the gated output in place, after flash_kernel (the decode kernels and prefill_kernel rotate in
-// their own epilogue).
-bn_status rotate_in_place(bn_ctx* ctx, hipStream_t st, const bn_attn_args* a) {
-    bn::RotateArgs r{};
-    r.attn = a->out;
-    r.a_ts = a->o_ts;
-    r.a_hs = a->o_hs;
-    r.signs = a->signs;
-    r.xr = a->out;
-    r.x_ts = a->o_ts;
-    r.x_hs = a->o_hs;
-    r.T = (int)a->T;
-    r.W = (int)a->H * bn::D;
-    bn_launch(ctx, bn::rotate_kernel, dim3(a->T, a->H / 2), dim3(64), 0, st, r);
-    return launched(ctx, "rotate_kernel");
-}
-
 // 17..64 rows that do not fill the GPU with prefill_kernel's q-tiles: verify_kernel over row groups of 8 rows (32
-// query rows of a kv head per block, q read once per key split) after append_kernel writes the rows. flash_kernel
-// has only one or two 32-token q-tiles per kv head there, so its parallelism comes from key splits that each reload
-// the q-tile and write 128 rows of partials: measured 16.5 against 30 us for 33 rows over 5 cached keys (8/2 heads)
-// and 36 against 71 us for 64 rows over 8,000 keys (16/4); from 100 rows up flash_kernel is faster (25 against
-// 30 us at 100 rows over 300 keys, 28 against 33 us at 256 over 512), since each of its blocks stages a K/V tile
-// once for 128 query rows where a row group uses it for 32. Keys per split: about kMidTargetBlocks blocks over the
-// kv heads and row groups, whole 32-key tiles for each of the W waves.
+// query rows of a kv head per block, q read once per key split) after append_kernel writes the rows. The q-tiles have
+// only one or two blocks per kv head there, and each of their key splits reloads the q-tile and writes 128 rows of
+// partials: a layer call of 17 rows over 300 keys measured 20.0 against 21.8 us (8/2 heads), of 20 over 5,000 25 against
+// 44 and of 64 over 8,000 43 against 54 (16/4); from 65 rows up the q-tiles take over (a row group uses a staged K/V
+// tile for 32 query rows where a q-tile uses it for 128). Keys per split: about kMidTargetBlocks blocks over the kv
+// heads and row groups, whole 32-key tiles for each of the W waves.
 constexpr int64_t kMidTargetBlocks = 256;
 constexpr uint32_t kMidMaxRows = 64;
 bool use_mid_rows(const bn_ctx* ctx, const bn_attn_args* a) {
@@ -681,7 +659,7 @@ size_t mid_records_bytes(const bn_attn_args* a) {
     return (size_t)(a->KV * 8 * T * ceil_div(ns, 8)) * bn::DEC_PART * sizeof(float);
 }
 
-bn_status run_flash(bn_ctx* ctx, hipStream_t st, const bn_attn_args* a) {
+bn_status run_tiles(bn_ctx* ctx, hipStream_t st, const bn_attn_args* a) {
     if (use_mid_rows(ctx, a)) {
         bn_attn_args m = *a;
         if (a->k_new) {
@@ -692,10 +670,13 @@ bn_status run_flash(bn_ctx* ctx, hipStream_t st, const bn_attn_args* a) {
         }
         return run_verify(ctx, st, &m, mid_chunk(a));
     }
-    const bool fused = use_prefill(a, ctx->prefill_min_blocks);  // prefill_kernel rotates in its epilogue
-    bn_status s = attend_flash(ctx, st, a);
-    if (s || !a->signs || fused) return s;
-    return rotate_in_place(ctx, st, a);
+    if (a->k_new) {
+        bn_status s = launch_append(ctx, st, a);
+        if (s) return s;
+    }
+    if (use_prefill(a, ctx->prefill_min_blocks)) return run_prefill(ctx, st, a, nullptr);
+    const SplitPlan p = plan_split(a->T, a->off, a->KV, ctx->split_target_blocks);
+    return run_prefill(ctx, st, a, &p);
 }
 
 // prep_kernel over the rows of p; kv_only: K/V cache rows only (the attention kernel norms and rotates q itself)
@@ -993,7 +974,7 @@ bn_status run(bn_ctx* ctx, hipStream_t st, const bn_attn_args* a, int kind) {
     else if (a->T == 1 || (kind != 3 && a->T <= (uint32_t)kVerifyMax))
         s = run_rows(ctx, st, a);
     else
-        s = run_flash(ctx, st, a);
+        s = run_tiles(ctx, st, a);
     return s ? s : launch_lora(ctx, st, a);
 }
 
@@ -1087,10 +1068,10 @@ bn_status bn_ctx_create(int device, bn_ctx** out) {
         const int v = atoi(e);
         if (v >= 1 && v <= kMaxSplitsCap) c->decode_max_splits = v;
     }
-    c->flash_target_blocks = (int)kFlashTargetBlocks;
+    c->split_target_blocks = (int)kSplitTarget;
     if (const char* e = getenv("BONSAI_ATTN_FLASH_TARGET_BLOCKS")) {
         const int v = atoi(e);
-        if (v >= 1 && v <= kFlashTargetBlocks) c->flash_target_blocks = v;
+        if (v >= 1 && v <= kSplitTarget) c->split_target_blocks = v;
     }
     c->verify_mfma = 1;
     if (const char* e = getenv("BONSAI_ATTN_VERIFY_MFMA")) c->verify_mfma = atoi(e) != 0;
@@ -1114,9 +1095,9 @@ size_t bn_attn_workspace_size(const bn_attn_args* a) {
     size_t rows = a->T <= (uint32_t)kVerifyMax ? plan_rows(a, 1, BN_DECODE_MAX_TARGET_WAVES, kMaxSplitsCap).total() : 0;
     if (verify_chunk(a)) rows = verify_q_offset(a) + (size_t)a->T * a->H * bn::D * sizeof(float);
     if (a->T == 1) return rows;
-    // the kernel choice for T >= 2 depends on the context, so the size covers the flash kernel's partials and, for
+    // the kernel choice for T >= 2 depends on the context, so the size covers the split key ranges' records and, for
     // more than 16 rows, verify_kernel's row-group records
-    size_t fl = plan_flash(a->T, a->off, a->KV).total();
+    size_t fl = plan_split(a->T, a->off, a->KV).total();
     if (a->T > (uint32_t)kVerifyMax && a->T <= kMidMaxRows) {
         const size_t mid = mid_records_bytes(a);
         if (mid > fl) fl = mid;
@@ -1368,7 +1349,7 @@ bn_status bn_attn_layer(bn_ctx* ctx, bn_stream stream, const bn_prep_args* p, co
     m.q_ts = p->q_ts;
     m.q_hs = p->q_hs;
     m.flags = p->flags;
-    s = run_flash(ctx, st, &m);
+    s = run_tiles(ctx, st, &m);
     return s ? s : launch_lora(ctx, st, &m);
 }
 

@@ -113,14 +113,6 @@ __device__ __forceinline__ int dec_len(const DecodeArgs& a, int i) {
 __device__ __forceinline__ int64_t dec_row0(const DecodeArgs& a, int i) {
     return a.kv_off ? a.kv_off[i] : a.row0 + (int64_t)i * a.row_step;
 }
-__device__ __forceinline__ int wave_incl_scan(int x, int lane) {
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o);
-        if (lane >= o) x += y;
-    }
-    return x;
-}
 __device__ __forceinline__ int64_t wave_sum64(int64_t x) {
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) x += __shfl_xor(x, o);
@@ -260,13 +252,6 @@ __device__ DecSplit dec_find_seq(const DecodeArgs& a, int seq, int lane) {
 __device__ __forceinline__ int64_t uniform64(int64_t x) {
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x), hi = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
     return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-
-// Wave-local LDS hand-off: the wave's LDS writes are complete and visible to its own lanes afterwards.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // W waves per block. A split's 16-key tiles are dealt to the waves in contiguous runs (wave w: tiles

@@ -74,6 +74,23 @@ __device__ __forceinline__ int call_off(const uint32_t* dyn, int off_max) {
     return off_max;
 }
 
+// Wave-local LDS hand-off: the wave's LDS writes are complete and visible to its own lanes afterwards.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// sums of x over the lanes up to this one
+__device__ __forceinline__ int wave_incl_scan(int x, int lane) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o);
+        if (lane >= o) x += y;
+    }
+    return x;
+}
+
 // reference gate: a * (1 / (1 + exp(-z)))  (gate_rotate.comp:19-22)
 __device__ __forceinline__ float gate_mul(float a, float z) { return a * (1.0f / (1.0f + expf(-z))); }
 // the same product on v_exp_f32 / v_rcp_f32 (about 2 ulp): for epilogues that gate many rows per lane

@@ -59,7 +59,17 @@ struct PrefillArgs {
                              // 2j, 2j+1, times the signs, Walsh-Hadamard transformed, / sqrt(512))
     const uint32_t* dyn;     // device offset (graph replay) or null; off is then its upper bound
     int T, off, KV, ntq;
+    // split key ranges (prefill_hilo_kernel<HILO, true>, then prefill_combine_kernel)
+    float* part_acc;         // [KV][ntq][max_splits][128 rows][256]
+    float* part_ml;          // [KV][ntq][max_splits][128 rows][2]: m (log2 domain), l
+    int ct, max_splits;      // key tiles per split at most, splits of a q-tile at most
+    int exact;               // prefill_hilo_kernel: key tiles from a range's start in which the running max is exact
 };
+
+constexpr int PF_ROWS = 4 * PF_BQ;        // query rows per q-tile
+
+// The splits of a q-tile over nt key tiles: n of them, split s takes tiles [s nt / n, (s + 1) nt / n)
+__host__ __device__ inline int pf_splits(int nt, int ct) { return (nt + ct - 1) / ct; }
 
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef short pf_s4v __attribute__((ext_vector_type(4)));

@@ -16,8 +16,14 @@
 //   - O stays in the accumulation registers for the whole loop.
 // Measured on MI355X (4096 rows, 16/4 heads): 248-282 us, against 171-178 us for prefill_kernel on the same rows
 // given as fp16 (the hi/lo product adds half again the MFMA work). Run on fp16 q, this design measured 194-226 us,
-// slower than prefill_kernel: one wave per SIMD issues LDS reads at about half the rate of two (130 against 260
-// bytes per cycle per CU for ds_read_b128), so fp16 q stays on prefill_kernel.
+// slower than prefill_kernel there: one wave per SIMD issues LDS reads at about half the rate of two (130 against 260
+// bytes per cycle per CU for ds_read_b128), so a long fp16 prefill stays on prefill_kernel.
+//
+// HILO = false is the same kernel on fp16 q, and SPLIT = true takes part of a q-tile's keys per block, for calls whose
+// q-tiles alone would leave CUs idle; prefill_combine_kernel merges the splits, gates and rotates. Against the kernel
+// with 64-key tiles, no pipelining and two separate launches for the merge and the rotation that these calls had (MI355X, a
+// layer call, fp32 q): 777 rows over 1,031, 16/4 heads 121 -> 71 us; 500 over 517, 8/2 53 -> 36; 1,900 over 4,000,
+// 16/4 492 -> 287; 3,000 over 1,000, 8/2 239 -> 161.
 #pragma once
 #include "bn_prefill.h"
 
@@ -42,6 +48,7 @@ constexpr int PH_OP = 1040;             // row pitch (bytes) of a wave's output 
 // 4-5% slower). Per tile the wave computes S^T(j + 1) = K(j + 1)
 // Q^T on the MFMA units while the VALU turns S^T(j) into P(j) (one k-step of each at a time), then O += P(j) V(j),
 // the operand reads a few MFMAs ahead of their use.
+template <bool HILO, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void prefill_hilo_kernel(PrefillArgs a) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[PH_STAGES * PF_STAGE];
     __shared__ f4 bc_lds[4][16];  // per wave: 64 floats broadcast in row order
@@ -51,9 +58,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const int h = lane >> 5, r32 = lane & 31;
     const int KV = a.KV, ntq = a.ntq;
 
-    // block -> (kv head, q-tile): longest q-tiles (highest index) first, each kv head on a fixed set of XCDs
-    int kh, qt;
-    {
+    // block -> (kv head, q-tile, split): longest q-tiles (highest index) first, each kv head on a fixed set of XCDs
+    int kh, qt, sp = 0;
+    const int off = call_off(a.dyn, a.off);
+    if constexpr (SPLIT) {
+        // the splits of the q-tiles, one after another, are a kv head's blocks: no block of the launch is without work
+        // (but past the last with a smaller device offset), and the XCDs get equal shares
+        const int idx = blockIdx.x / KV;
+        kh = blockIdx.x % KV;
+        qt = -1;
+        for (int c = 0, base = 0; c < ntq; c += 64) {
+            const int q = ntq - 1 - c - lane;
+            const int n = q < 0 ? 0 : pf_splits((off + min(a.T, (q + 1) * PF_BQ) - 1 + PF_BK) / PF_BK, a.ct);
+            const int incl = wave_incl_scan(n, lane);
+            const uint64_t hit = __ballot(base + incl > idx);
+            if (hit) {
+                const int f = __builtin_ctzll(hit);
+                qt = ntq - 1 - c - f;
+                sp = idx - base - __builtin_amdgcn_readlane(incl - n, f);
+                break;
+            }
+            base += __builtin_amdgcn_readlane(incl, 63);
+        }
+        if (qt < 0) return;
+        qt = __builtin_amdgcn_readfirstlane(qt);
+        sp = __builtin_amdgcn_readfirstlane(sp);
+    } else {
         const int b = blockIdx.x, nb = KV * ntq;
         int idx;
         if (8 % KV == 0 && nb % 8 == 0) {
@@ -68,41 +98,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     }
     const int t0 = qt * PF_BQ;
     const int t_last = min(a.T, t0 + PF_BQ) - 1;
-    const int off = call_off(a.dyn, a.off);
     const int nk = off + a.T;                         // cache rows that exist
-    const int nt = (off + t_last + PF_BK) / PF_BK;    // key tiles the q-tile attends to
+    const int nt_all = (off + t_last + PF_BK) / PF_BK;  // key tiles the q-tile attends to
+    // the block's key tiles [jb, nt)
+    int jb = 0, nt = nt_all;
+    if constexpr (SPLIT) {
+        const int n = pf_splits(nt_all, a.ct);
+        jb = (int)((int64_t)sp * nt_all / n);
+        nt = (int)((int64_t)(sp + 1) * nt_all / n);
+    }
     const int64_t kvd = (int64_t)KV * D;
     const uint16_t* kb = a.kc + (int64_t)kh * D;
     const uint16_t* vb = a.vc + (int64_t)kh * D;
     const int head = kh * 4 + w;
-
-    // Q^T hi and lo straight from memory, before the copies (which count on the same vmcnt): lane l holds token
-    // t0 + l % 32 (clamped), dims 16 ks + 8 h .. +7
-    h8 qb[16], ql[16];
-    {
-        const int tq = min(t0 + r32, a.T - 1);
-        const float* qr = a.q + (int64_t)tq * a.q_ts + (int64_t)head * a.q_hs + 8 * h;
-#pragma unroll
-        for (int ks = 0; ks < 16; ks++) {
-            const f4 x0 = *reinterpret_cast<const f4*>(qr + 16 * ks);
-            const f4 x1 = *reinterpret_cast<const f4*>(qr + 16 * ks + 4);
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const float x = e < 4 ? x0[e] : x1[e - 4];
-                const _Float16 hi = (_Float16)x;
-                qb[ks][e] = hi;
-                ql[ks][e] = (_Float16)(x - (float)hi);
-            }
-        }
-    }
-    // The loads have landed; the empty asm statements then redefine Q^T, so the compiler's own waits for these loads
-    // (which would count the tile copies issued next) end here.
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-    for (int ks = 0; ks < 16; ks++) {
-        asm volatile("" : "+v"(qb[ks]));
-        asm volatile("" : "+v"(ql[ks]));
-    }
 
     // Tile copies: wave w moves row pairs 4w .. 4w+3 of K and of V (8 copies per tile); copy c of tile jt: K (c even)
     // or V (c odd) of row pair 4 w + c / 2, lane l loading row 32 jt + p + 16 (l / 32), clamped to the cache's last row
@@ -115,12 +123,71 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         else
             pf_copy16(reinterpret_cast<const char*>(kb + (int64_t)j0 * kvd) + go, st + p * PF_KP);
     };
-    // tiles 0, 1, 2 into stages 0, 1, 2 (a tile past the last repeats the last: its stage is never read as such), so
-    // that every tile step finds the same copies in flight
+    // tiles jb, jb + 1, jb + 2 into stages 0, 1, 2 (a tile past the last repeats the last: its stage is never read as
+    // such), so that every tile step finds the same copies in flight
 #pragma unroll
     for (int j = 0; j < PH_STAGES - 1; j++)
 #pragma unroll
-        for (int c = 0; c < 8; c++) tile_copy(min(j, nt - 1), lds + j * PF_STAGE, c);
+        for (int c = 0; c < 8; c++) tile_copy(min(jb + j, nt - 1), lds + j * PF_STAGE, c);
+
+    // Q^T (hi and lo), under the copies' latency: lane l holds token t0 + l % 32 (clamped), dims 16 ks + 8 h .. +7. Read
+    // straight into that layout every load touches 64 places (64 cycles of the address unit each, 128 loads of fp32 per
+    // CU: 4 us of a block's start), so four neighbouring lanes read 64 bytes of a row and the wave turns 256 bytes of its
+    // 32 rows at a time in LDS (stage 3, free until the first tile step): 16-byte slot s of row r at
+    // s ^ 4 (r % 4) ^ (r / 4) % 4, which keeps the writes (4 rows x 4 slots) and the reads (16 rows) on distinct banks.
+    h8 qb[16], ql[HILO ? 16 : 1];
+    {
+        constexpr int NP = HILO ? 4 : 2, ES = HILO ? 4 : 2;
+        u4 raw[NP][4][2];
+#pragma unroll
+        for (int rh = 0; rh < 2; rh++) {
+            const int tq = min(t0 + (lane >> 2) + 16 * rh, a.T - 1);
+            const char* qr = (HILO ? reinterpret_cast<const char*>(a.q) : reinterpret_cast<const char*>(a.q16)) +
+                             ((int64_t)tq * a.q_ts + (int64_t)head * a.q_hs) * ES + 16 * (lane & 3);
+#pragma unroll
+            for (int p = 0; p < NP; p++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) raw[p][g][rh] = *reinterpret_cast<const u4*>(qr + 256 * p + 64 * g);
+        }
+        uint8_t* const qs = lds + (PH_STAGES - 1) * PF_STAGE + w * 8192;
+        auto slot = [&](int r, int s) { return qs + r * 256 + 16 * (s ^ (4 * (r & 3)) ^ ((r >> 2) & 3)); };
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+#pragma unroll
+                for (int rh = 0; rh < 2; rh++)
+                    *reinterpret_cast<u4*>(slot((lane >> 2) + 16 * rh, 4 * g + (lane & 3))) = raw[p][g][rh];
+            wave_lds_sync();
+            if constexpr (HILO) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const int ks = 4 * p + k;
+                    const f4 x0 = *reinterpret_cast<const f4*>(slot(r32, 4 * k + 2 * h));
+                    const f4 x1 = *reinterpret_cast<const f4*>(slot(r32, 4 * k + 2 * h + 1));
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        const float x = e < 4 ? x0[e] : x1[e - 4];
+                        const _Float16 hi = (_Float16)x;
+                        qb[ks][e] = hi;
+                        ql[ks][e] = (_Float16)(x - (float)hi);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < 8; k++) qb[8 * p + k] = *reinterpret_cast<const h8*>(slot(r32, 2 * k + h));
+            }
+            wave_lds_sync();
+        }
+    }
+    // The loads have landed (and the copies before them); the empty asm statements then redefine Q^T, so the compiler's
+    // own waits for these loads (which would count the tile copies issued next) end here.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int ks = 0; ks < 16; ks++) {
+        asm volatile("" : "+v"(qb[ks]));
+        if constexpr (HILO) asm volatile("" : "+v"(ql[ks]));
+    }
 
     f16x o[8];
 #pragma unroll
@@ -135,8 +202,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const int v_lane = PF_KB + (4 * h + (vs >> 2)) * PF_VP + 32 * vnh + 8 * (vs & 3);
     float* bc = reinterpret_cast<float*>(bc_lds[w]);
 
-    // tile 0 landed (tiles 1 and 2 may still be in flight), for every wave; then S^T(0)
-    asm volatile("s_waitcnt vmcnt(16)\n\ts_barrier" ::: "memory");
+    // the first tiles landed for every wave; then S^T of the first
+    asm volatile("s_barrier" ::: "memory");
     f16x s_cur;
     {
         const uint8_t* kl = lds + k_lane;
@@ -146,20 +213,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         for (int ks = 0; ks < 16; ks++) {
             const h8 kop = pf_lds_h8(kl + ks * 32);
             s_cur = mfma32(kop, qb[ks], s_cur);
-            s_cur = mfma32(kop, ql[ks], s_cur);
+            if constexpr (HILO) s_cur = mfma32(kop, ql[ks], s_cur);
         }
     }
 
     // Tile j: S^T(j + 1) from stage j + 1 (computed also after the last tile, from a stage whose copies are done,
     // and dropped), P(j) from S^T(j), O += P(j) V(j) from stage j.
-    for (int j = 0; j < nt; j++) {
+    for (int j = jb; j < nt; j++) {
         // tile j + 1 landed (tile j + 2's copies may be in flight), and every wave is done with tile j - 1, whose
         // stage takes tile j + 3 (a repeat of the last tile past the end), copied during the S^T(j + 1) MFMAs below
         asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
-        const int jc = min(j + 3, nt - 1);
-        uint8_t* cst = lds + ((j + 3) & (PH_STAGES - 1)) * PF_STAGE;
-        const uint8_t* cur = lds + (j & (PH_STAGES - 1)) * PF_STAGE;
-        const uint8_t* nxt = lds + ((j + 1) & (PH_STAGES - 1)) * PF_STAGE;
+        const int jc = min(j + 3, nt - 1), js = j - jb;
+        uint8_t* cst = lds + ((js + 3) & (PH_STAGES - 1)) * PF_STAGE;
+        const uint8_t* cur = lds + (js & (PH_STAGES - 1)) * PF_STAGE;
+        const uint8_t* nxt = lds + ((js + 1) & (PH_STAGES - 1)) * PF_STAGE;
 
         // K(j + 1) operand reads run KA k-steps ahead of their MFMAs; the first ones hide behind the row max
         constexpr int KA = PH_KAHEAD, VA = PH_VAHEAD;
@@ -184,10 +251,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         const float tmax = tm * sc;  // log2 domain
         // Conditional rescale: m_run moves only when the row's tile max exceeds it by more than 8 (log2 units);
         // otherwise p = 2^(x - m_run) <= 256 stays well inside fp16 and the final division by l cancels the common
-        // factor. Rows with no key yet (m_run = -inf) have O = 0 and just take the max.
+        // factor. Rows with no key yet (m_run = -inf) have O = 0 and just take the max. In the first
+        // a.exact tiles m_run follows the max exactly: the weight of a row's largest key so far is then 1, which fp16
+        // holds exactly, and in a short range those weights carry the rounding error (128 keys: 1.6e-4 of the output
+        // instead of 1.9e-4). O's rescale costs about a third of a tile.
         float alpha = 1.0f;
         bool moved = false;
-        if (tmax > m_run + 8.0f) {
+        if (tmax > m_run + (j - jb < a.exact ? 0.0f : 8.0f)) {
             moved = m_run != -INFINITY;
             alpha = moved ? __builtin_amdgcn_exp2f(m_run - tmax) : 0.0f;
             m_run = tmax;
@@ -229,12 +299,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             if (ks + KA < 16) kop[ks + KA] = pf_lds_h8(kl + (ks + KA) * 32);
             if (ks + VA >= 16) v_read(ks + VA - 16);
             s_next = mfma32(kop[ks], qb[ks], s_next);
-            s_next = mfma32(kop[ks], ql[ks], s_next);
+            if constexpr (HILO) s_next = mfma32(kop[ks], ql[ks], s_next);
             pa[ks >> 3][ks & 7] = (_Float16)__builtin_amdgcn_exp2f(fmaf(s_cur[ks], sc, -m_use));
             if (ks + KA < 16 && ks + VA >= 16) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
             else if (ks + KA < 16) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             else if (ks + VA >= 16) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, HILO ? 2 : 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x402, 4, 0);
             if (ks & 1) {  // one copy after every second k-step's MFMAs, which stay ahead of it
                 tile_copy(jc, cst, ks >> 1);
@@ -263,9 +333,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     }
 
     // Epilogue. O / l goes to LDS as each wave's [32 tokens][256 dims] (pitch PH_OP), then rows are read back 16
-    // bytes per lane for coalesced gated stores, or, with signs, per (token, head pair) for the rotation.
+    // bytes per lane for coalesced gated stores, or, with signs, per (token, head pair) for the rotation. A wave's rows
+    // are head w's 32 tokens, or (rotated) head pair w % 2 of the tokens w / 2 + 2 k; their gate rows are all requested
+    // here: read row by row between the stores (which may alias them) they cost a round trip each, 16 or 8 in a row on a CU
+    // that runs nothing else (4,096 rows, 16/4 heads: 249 against 233 us; 70 rows rotated, 8/2: 31 against 20).
+    f4 z[32], sg[2];
+    if constexpr (!SPLIT) {
+        if (a.gate) {
+#pragma unroll
+            for (int k = 0; k < 32; k++) {
+                const int tl = a.signs ? (w >> 1) + 2 * (k >> 1) : k;
+                const int hd = a.signs ? kh * 4 + 2 * (w & 1) + (k & 1) : head;
+                z[k] = *reinterpret_cast<const f4*>(a.gate + (int64_t)min(t0 + tl, a.T - 1) * a.g_ts +
+                                                    (int64_t)hd * a.g_hs + 4 * lane);
+            }
+        }
+        if (a.signs)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                sg[i] = *reinterpret_cast<const f4*>(a.signs + (int64_t)(kh * 4 + 2 * (w & 1) + i) * D + 4 * lane);
+    }
     const float l_tot = sum_xhalf(l_run);
-    if (h == 0) bc[r32] = 1.0f / l_tot;
+    if (h == 0) bc[r32] = SPLIT ? 1.0f : 1.0f / l_tot;
     f4 lv[4];
 #pragma unroll
     for (int gg = 0; gg < 4; gg++) lv[gg] = bc_lds[w][2 * gg + h];
@@ -280,48 +369,164 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             *reinterpret_cast<float*>(orow + tl * PH_OP + 4 * (32 * dt + r32)) = o[dt][r] * lv[r >> 2][r & 3];
         }
     __syncthreads();
-    if (!a.signs) {
+    if constexpr (SPLIT) {
+        // the split's record: unnormalised rows, m and l per row
+        const int64_t row = (((int64_t)kh * ntq + qt) * a.max_splits + sp) * PF_ROWS + w * PF_BQ;
+        if (h == 0) {
+            a.part_ml[(row + r32) * 2] = m_run;
+            a.part_ml[(row + r32) * 2 + 1] = l_tot;
+        }
 #pragma unroll 4
+        for (int tl = 0; tl < PF_BQ; tl++)
+            *reinterpret_cast<f4*>(a.part_acc + (row + tl) * D + 4 * lane) =
+                *reinterpret_cast<const f4*>(orow + tl * PH_OP + 16 * lane);
+        return;
+    }
+    if (!a.signs) {
+#pragma unroll
         for (int tl = 0; tl < PF_BQ; tl++) {
             const int t = t0 + tl;
-            if (t >= a.T) break;
             f4 y = *reinterpret_cast<const f4*>(orow + tl * PH_OP + 16 * lane);
             if (a.gate) {
-                const f4 z = *reinterpret_cast<const f4*>(a.gate + (int64_t)t * a.g_ts + (int64_t)head * a.g_hs + 4 * lane);
 #pragma unroll
-                for (int e = 0; e < 4; e++) y[e] = gate_mul_fast(y[e], z[e]);
+                for (int e = 0; e < 4; e++) y[e] = gate_mul_fast(y[e], z[tl][e]);
             }
-            __builtin_nontemporal_store(y, reinterpret_cast<f4*>(a.out + (int64_t)t * a.o_ts + (int64_t)head * a.o_hs +
-                                                               4 * lane));  // streamed out, as in prefill_kernel
+            if (t < a.T)
+                __builtin_nontemporal_store(y, reinterpret_cast<f4*>(a.out + (int64_t)t * a.o_ts +
+                                                                   (int64_t)head * a.o_hs + 4 * lane));
         }
         return;
     }
-    // rotation: (token tl, head pair p) blocks, 16 per wave; lane l holds dims 4l .. 4l+3 of heads 2p and 2p + 1
-#pragma unroll 1
-    for (int k = w; k < 2 * PF_BQ; k += 4) {
-        const int tl = k >> 1, p = k & 1, t = t0 + tl;
-        if (t >= a.T) break;
+    // rotation: lane l holds dims 4l .. 4l+3 of heads 2p and 2p + 1
+    const int p = w & 1;
+#pragma unroll
+    for (int k = 0; k < PF_BQ / 2; k++) {
+        const int tl = (w >> 1) + 2 * k, t = t0 + tl;
         float v[8];
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-            const int hw = 2 * p + i, hd = kh * 4 + hw;
-            f4 y = *reinterpret_cast<const f4*>(lds + hw * 32 * PH_OP + tl * PH_OP + 16 * lane);
+            f4 y = *reinterpret_cast<const f4*>(lds + (2 * p + i) * 32 * PH_OP + tl * PH_OP + 16 * lane);
             if (a.gate) {
-                const f4 z = *reinterpret_cast<const f4*>(a.gate + (int64_t)t * a.g_ts + (int64_t)hd * a.g_hs + 4 * lane);
 #pragma unroll
-                for (int e = 0; e < 4; e++) y[e] = gate_mul_fast(y[e], z[e]);
+                for (int e = 0; e < 4; e++) y[e] = gate_mul_fast(y[e], z[2 * k + i][e]);
             }
-            y *= *reinterpret_cast<const f4*>(a.signs + (int64_t)hd * D + 4 * lane);
+            y *= sg[i];
 #pragma unroll
             for (int c = 0; c < 4; c++) v[4 * i + c] = y[c];
         }
         fwht512_wave(v, lane);
         float* o_ = a.out + (int64_t)t * a.o_ts + (int64_t)(kh * 4 + 2 * p) * a.o_hs;
+        if (t < a.T)
 #pragma unroll
-        for (int i = 0; i < 2; i++)
-            __builtin_nontemporal_store(f4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]} * INV_SQRT512,
-                                        reinterpret_cast<f4*>(o_ + i * a.o_hs + 4 * lane));
+            for (int i = 0; i < 2; i++)
+                __builtin_nontemporal_store(f4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]} * INV_SQRT512,
+                                            reinterpret_cast<f4*>(o_ + i * a.o_hs + 4 * lane));
     }
+}
+
+// Merge of the key splits of one (token, head pair) in split order (attn_combine.comp:10-20), then the gate and, with
+// signs, the rotation of the pair's 512 elements (gate_rotate.comp:18-25). Grid (T, H / 2) x 64 threads; thread: dims
+// 4 lane .. +3 of both heads. Bound by the records' round trips: the first 8 splits' accumulators are requested with
+// the (m, l) terms.
+__global__ __launch_bounds__(64) void prefill_combine_kernel(PrefillArgs a) {
+    constexpr int PRE = 8;
+    const int t = blockIdx.x, lane = threadIdx.x, kh = blockIdx.y >> 1, p = blockIdx.y & 1;
+    const int qt = t / PF_BQ, t_last = min(a.T, qt * PF_BQ + PF_BQ) - 1;
+    const int hd = kh * 4 + 2 * p;  // the pair's first head
+    f4 z[2], sg[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        z[i] = sg[i] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (a.gate)
+            z[i] = *reinterpret_cast<const f4*>(a.gate + (int64_t)t * a.g_ts + (int64_t)(hd + i) * a.g_hs + 4 * lane);
+        if (a.signs) sg[i] = *reinterpret_cast<const f4*>(a.signs + (int64_t)(hd + i) * D + 4 * lane);
+    }
+    const int ns = pf_splits((call_off(a.dyn, a.off) + t_last + PF_BK) / PF_BK, a.ct);
+    // row of split 0, head 2 p; head i is PF_BQ rows on, split s PF_ROWS rows
+    const int64_t row0 = ((int64_t)kh * a.ntq + qt) * a.max_splits * PF_ROWS + 2 * p * PF_BQ + t % PF_BQ;
+    auto acc_of = [&](int s, int i) {
+        return *reinterpret_cast<const f4*>(a.part_acc + (row0 + (int64_t)s * PF_ROWS + i * PF_BQ) * D + 4 * lane);
+    };
+    f4 pre[PRE][2];
+#pragma unroll
+    for (int u = 0; u < PRE; u++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) pre[u][i] = u < ns ? acc_of(u, i) : f4{0.0f, 0.0f, 0.0f, 0.0f};
+    float y[8];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const float* ml = a.part_ml + (row0 + i * PF_BQ) * 2;
+        float L = 0.0f;
+        f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (ns <= PRE) {
+            // few splits: every lane takes all their terms, without the exchanges below
+            float m[PRE], l[PRE];
+#pragma unroll
+            for (int u = 0; u < PRE; u++) {
+                const float* r = ml + (int64_t)min(u, ns - 1) * PF_ROWS * 2;
+                m[u] = u < ns ? r[0] : -INFINITY;
+                l[u] = r[1];
+            }
+            float M = m[0];
+#pragma unroll
+            for (int u = 1; u < PRE; u++) M = fmaxf(M, m[u]);
+#pragma unroll
+            for (int u = 0; u < PRE; u++) {
+                const float wu = m[u] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[u] - M);
+                L = fmaf(l[u], wu, L);
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[e] = fmaf(pre[u][i][e], wu, acc[e]);
+            }
+        } else {
+            auto m_of = [&](int s) { return s < ns ? ml[(int64_t)s * PF_ROWS * 2] : -INFINITY; };
+            const float m0 = m_of(lane), l0 = lane < ns ? ml[(int64_t)lane * PF_ROWS * 2 + 1] : 0.0f;
+            float M = m0;
+            for (int s = lane + 64; s < ns; s += 64) M = fmaxf(M, m_of(s));
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
+            for (int base = 0; base < ns; base += 64) {
+                const int s_ = base + lane;
+                float ms = m0, ls = l0;
+                if (base > 0) {
+                    ms = m_of(s_);
+                    ls = s_ < ns ? ml[(int64_t)s_ * PF_ROWS * 2 + 1] : 0.0f;
+                }
+                const float wgt = ms == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms - M);  // split base + lane
+                const int cnt = min(64, ns - base);
+                auto add = [&](int u, f4 v) {
+                    const float wu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), u));
+                    L = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(ls), u)), wu, L);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[e] = fmaf(v[e], wu, acc[e]);
+                };
+                int u0 = 0;
+                if (base == 0) {
+#pragma unroll
+                    for (int u = 0; u < PRE; u++)
+                        if (u < cnt) add(u, pre[u][i]);
+                    u0 = PRE;
+                }
+                for (; u0 < cnt; u0++) add(u0, acc_of(base + u0, i));
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            float v = acc[e] / L;
+            if (a.gate) v = gate_mul(v, z[i][e]);
+            y[4 * i + e] = v;
+        }
+    }
+    float* o = a.out + (int64_t)t * a.o_ts + (int64_t)hd * a.o_hs + 4 * lane;
+    float scale = 1.0f;
+    if (a.signs) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) y[e] *= sg[e >> 2][e & 3];
+        fwht512_wave(y, lane);
+        scale = INV_SQRT512;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+        *reinterpret_cast<f4*>(o + i * a.o_hs) = f4{y[4 * i], y[4 * i + 1], y[4 * i + 2], y[4 * i + 3]} * scale;
 }
 
 }  // namespace bn
