@@ -177,8 +177,8 @@ DecodePlan plan_rows(const bn_attn_args* a, int64_t waves, int64_t target_waves,
 // T >= 2 rows: q-tiles of 32 tokens of the 4 query heads of a kv head, one block each (prefill_hilo_kernel: one block per
 // CU, so kSplitTarget blocks run at once). When the q-tiles alone leave CUs idle, each q-tile's key tiles are cut into
 // ceil(nt / ct) equal splits, ct the least number that gives no more blocks than that: a block costs a start (q rows,
-// the first tiles, about 4 us) and a 128 KB record besides about 2 us per key tile, so a second round of blocks loses
-// more than it balances (777 rows over 1,031, 16/4 heads: 44 us a call in one round, 60 with the XCDs' shares uneven).
+// the first tiles) and a 128 KB record besides about 2 us per key tile, so a second round of blocks loses more than it
+// balances (a layer call of 777 rows over 1,031, 16/4 heads: 67 us in one round, 85 with uneven shares for the XCDs).
 // At least 3 tiles a split, or 2 where that gives no more than half the blocks (256 rows over 512, 8/2 heads: 25.1
 // with 3, 26.0 with 4, 27.9 with 6; a layer call of 70 rows over none: 23.7 with 2, 28.2 unsplit). Depends only on the
 // shapes.

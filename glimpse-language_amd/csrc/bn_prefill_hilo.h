@@ -21,8 +21,8 @@
 //
 // HILO = false is the same kernel on fp16 q, and SPLIT = true takes part of a q-tile's keys per block, for calls whose
 // q-tiles alone would leave CUs idle; prefill_combine_kernel merges the splits, gates and rotates. Against the kernel
-// with 64-key tiles, no pipelining and two separate launches for the merge and the rotation that these calls had (MI355X, a
-// layer call, fp32 q): 777 rows over 1,031, 16/4 heads 121 -> 71 us; 500 over 517, 8/2 53 -> 36; 1,900 over 4,000,
+// with 64-key tiles, no pipelining and two separate launches for the merge and the rotation that these calls had
+// (MI355X, a layer call, fp32 q): 777 rows over 1,031, 16/4 heads 121 -> 71 us; 500 over 517, 8/2 53 -> 36; 1,900 over 4,000,
 // 16/4 492 -> 287; 3,000 over 1,000, 8/2 239 -> 161.
 #pragma once
 #include "bn_prefill.h"
@@ -130,11 +130,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 #pragma unroll
         for (int c = 0; c < 8; c++) tile_copy(min(jb + j, nt - 1), lds + j * PF_STAGE, c);
 
-    // Q^T (hi and lo), under the copies' latency: lane l holds token t0 + l % 32 (clamped), dims 16 ks + 8 h .. +7. Read
-    // straight into that layout every load touches 64 places (64 cycles of the address unit each, 128 loads of fp32 per
-    // CU: 4 us of a block's start), so four neighbouring lanes read 64 bytes of a row and the wave turns 256 bytes of its
+    // Q^T (hi and lo), under the copies' latency: lane l holds token t0 + l % 32 (clamped), dims 16 ks + 8 h .. +7.
+    // Read straight into that layout every load touches 64 places (64 cycles of the address unit each, 128 loads of fp32 per
+    // CU, at every block's start), so four neighbouring lanes read 64 bytes of a row and the wave turns 256 bytes of its
     // 32 rows at a time in LDS (stage 3, free until the first tile step): 16-byte slot s of row r at
-    // s ^ 4 (r % 4) ^ (r / 4) % 4, which keeps the writes (4 rows x 4 slots) and the reads (16 rows) on distinct banks.
+    // s ^ 4 (r % 4) ^ (r / 4) % 4, which keeps the writes (4 rows x 4 slots) and the reads (16 rows) on distinct banks
+    // (256 rows over 512, 8/2 heads: 26.4 -> 25.7 us).
     h8 qb[16], ql[HILO ? 16 : 1];
     {
         constexpr int NP = HILO ? 4 : 2, ES = HILO ? 4 : 2;
@@ -335,8 +336,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // Epilogue. O / l goes to LDS as each wave's [32 tokens][256 dims] (pitch PH_OP), then rows are read back 16
     // bytes per lane for coalesced gated stores, or, with signs, per (token, head pair) for the rotation. A wave's rows
     // are head w's 32 tokens, or (rotated) head pair w % 2 of the tokens w / 2 + 2 k; their gate rows are all requested
-    // here: read row by row between the stores (which may alias them) they cost a round trip each, 16 or 8 in a row on a CU
-    // that runs nothing else (4,096 rows, 16/4 heads: 249 against 233 us; 70 rows rotated, 8/2: 31 against 20).
+    // here: read row by row between the stores (which may alias them) they cost a round trip each, 16 or 8 in a row on a
+    // CU that runs nothing else (a layer call of 4,096 rows, 16/4 heads: 276 against 257 us; of 70 rows, 8/2: 31 against
+    // 27).
     f4 z[32], sg[2];
     if constexpr (!SPLIT) {
         if (a.gate) {
