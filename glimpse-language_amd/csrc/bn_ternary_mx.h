@@ -6,15 +6,25 @@
 //   W: a code c becomes the fp4 value 2 (c - 1) in {-2, 0, 2, 4}; the row's fp16 scale multiplies the sum of each
 //      128-column group in fp32 afterwards (as qmv.glsl:22-35 does), one fma per output and group.
 //   x: 32 columns of a token share the power of two S = 2^floor(log2(max |x|)), and x is written as five fp6 (e2m3)
-//      digits, x = S (n0 + n1 / 32 + ... + n4 / 32^4) / 8 with whole n_i in -16..16 (each the nearest to what the
-//      digits before it left, so exact differences), to within S 2^-24: fp32's own last bit for the block's largest
-//      value. The digit's power of two is the instruction's block scale, so one fp32 accumulator takes all five
-//      (smallest first), and a group's products are summed without a rounding between its columns' scales.
+//      digits, x = S / 2 (q0 + q1 / 32 + ... + q4 / 32^4), each the fp6 value nearest to what the digits before it left
+//      (|q| <= 4, in steps of 1/8 up to 2 and of 1/4 above: exact differences), to within S 2^-25 for most values and
+//      S 2^-24 for all: fp32's own last bit for the block's largest. The digit's power of two is the instruction's block
+//      scale, so one fp32 accumulator takes all five (smallest first), and a group's products are summed without a
+//      rounding between its columns' scales.
 //   Five MFMAs per 64 columns thus replace the eight of an fp16 hi/lo split, at the same time each.
-// A block of 32 values whose largest is far above the rest (sum |x| < 4 max |x|, and digits that do not end) would
-// leave the small ones with fewer bits than fp32 has: its remainder is written as five more digits and multiplied by
-// a second pass over the group (flagged per 32-token tile; blocks that need none are zero there). The block scale
-// covers fp32's exponents; a block whose sum of |x| is not finite gets the scale NaN, and the token's outputs are NaN.
+// Digits end at the same place for all 32 values, so columns far below a block's largest keep fewer bits of their own,
+// which a row whose weights are 0 on the large columns shows. Such a block's remainder is written as five more digits and
+// multiplied by a second pass over the group (flagged per 32-token tile; blocks that need none are zero there). It is
+// made where the digits of these columns do not end:
+//   - at least 12 of the block's columns within S 2^-5, 7 within S 2^-7 or 4 within S 2^-10; or
+//   - a column within S 2^-5 in every token of the tile (of 8 tokens or more), as columns of another scale are.
+// With small columns in the same places for a tile's tokens their error is then at most 1e-6 of their norm, and 2.2e-6
+// for single tokens with up to 25 large columns of 32 (worst of 1 to 31 large columns, 8 to 10^5 times the others, weights
+// 0 under them; the digits alone: 3e-3). The rules are no wider because a step with a second pass takes more than
+// twice as long, and the blocks of a call that runs in one round wait for it: they take 2e-7 of the blocks of normally
+// distributed values for such (with 6 and 3 in the places of 7 and 4 it was 2e-5, and calls of 1,000 to 2,000 tokens
+// took 10-20% longer). The block scale covers fp32's exponents; a block with an infinity or a NaN gets the scale NaN,
+// and the token's outputs are NaN.
 // Measured (MI355X, the 4B q/k/v projections of 4,096 tokens): 303 us (digits 17, GEMM 285) against 368 for the fp16
 // hi/lo split, whose 1.16 PFLOP/s of products were the rate of a large library product here; error against 64-bit sums
 // 1.1e-7 of the output's norm against 4.6e-7. The matrix units are busy two thirds of the time at the 1.7 GHz that the
@@ -41,7 +51,8 @@ constexpr int TMX_G = 128;                      // columns per group (one weight
 constexpr int TMX_ND = 5;                       // digits
 constexpr int TMX_FRAG = 64 * 48;               // bytes of a digit: per lane 12 words (kh = 0, then 1) in three 1 KB planes
 constexpr int TMX_DIG = TMX_ND * TMX_FRAG;      // 15,360
-constexpr int TMX_TILE = TMX_DIG + 256;         // a 32-token tile of a group: fragments, then per lane the two scale bytes
+// a 32-token tile of a group: fragments, then per lane the scale bytes of its two blocks and whether each is wide
+constexpr int TMX_TILE = TMX_DIG + 256;
 
 // 32-token tiles of a call (an even number: the blocks take two)
 __host__ __device__ inline int tern_mx_tiles(int T) { return 2 * ((T + 63) / 64); }
@@ -51,29 +62,74 @@ inline size_t tern_pf_work_bytes(int T, int K) {
 }
 static_assert(2 * (TMX_TILE + 4) <= 2 * (16384 + 4), "the workspace holds the tiles and their flags");
 
-// The digits of 32 values of a token. In: x by element (u[i] = element 2 i, v[i] = element 2 i + 1). Out: each
-// digit's six words through put(d, words), the remainders in u and v, whether they need a second set of digits in wide;
-// returns the block's scale byte.
 struct TernBlock {
-    f16x u, v;
+    f16x u, v;  // 32 values of a token by element: u[i] = element 2 i, v[i] = element 2 i + 1
 };
 __device__ __forceinline__ float tern_pow2(int e) { return __int_as_float(e << 23); }
-template <typename Put>
-__device__ __forceinline__ int tern_digits(TernBlock& x, bool& wide, const Put& put) {
-    float mx = 0.0f, sum = 0.0f;  // an infinity or a NaN shows in the sum (as do finite values whose sum overflows)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(mx) : "v"(x.u[i]), "v"(x.v[i]));
-        sum += fabsf(x.u[i]) + fabsf(x.v[i]);
+// word i of 16 six-bit fields of value f in three words
+__host__ __device__ constexpr uint32_t tern_fields(uint32_t f, int i) {
+    uint32_t r = 0;
+    for (int j = 0; j < 16; ++j) {
+        const int at = 6 * j - 32 * i;
+        if (at > -6 && at < 32) r |= at >= 0 ? f << at : f >> -at;
     }
-    const int e = sum < INFINITY ? max(__float_as_int(mx) >> 23, 28) : 255;  // 28: the last digit's scale stays normal
-    const bool spread = sum < 4.0f * mx;  // the largest value far above the rest
+    return r;
+}
+// Which of a digit's 32 values are at least Q eighths: a code's magnitude (6 bits: sign, magnitude) plus 32 - Q carries
+// into the sign's place if it is. The 16 such places of three words fall on distinct odd bits: bit tern_bit(e) of the
+// result is element e.
+template <int Q>
+__device__ __forceinline__ uint32_t tern_at_least(u6v w) {
+    uint32_t r[2] = {0, 0};
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        uint32_t carry = 0;
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            r[half] |= __builtin_addc(w[3 * half + i] & tern_fields(31, i), tern_fields(32 - Q, i), carry, &carry) &
+                       tern_fields(32, i);
+    }
+    return r[0] | (r[1] >> 1);
+}
+__host__ __device__ constexpr int tern_bit(int e) { return (6 * (e & 15) + 5) % 32 - (e >> 4); }
+// OR over the 32 lanes of a lane's half
+__device__ __forceinline__ uint32_t or_half(uint32_t x) {
+    x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xF, 0xF, false);  // row_ror: 8, 4, 2, 1
+    x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x124, 0xF, 0xF, false);
+    x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x122, 0xF, 0xF, false);
+    x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x121, 0xF, 0xF, false);
+    const auto p = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    return p[0] | p[1];
+}
+// The digits of 32 values x of a token: each digit's six words through put(d, words). Returns the block's scale byte.
+// CHECK = false: x becomes the remainders. CHECK = true also tells in wide whether the block needs a second set of
+// digits (zeros for tokens past T; many: whether the tile has 8 tokens or more, lane: token lane % 32 of it).
+template <bool CHECK, typename Put>
+__device__ __forceinline__ int tern_digits(TernBlock& x, bool many, bool& wide, const Put& put) {
+    float mx = 0.0f;  // an infinity or a NaN stays
+#pragma unroll
+    for (int i = 0; i < 16; ++i) asm("v_maximum3_f32 %0, |%1|, |%2|, %0" : "+v"(mx) : "v"(x.u[i]), "v"(x.v[i]));
+    const int eb = (__float_as_int(mx) >> 23) & 255;
+    const int e = max(eb - 1, 28);  // 28: the last digit's scale stays normal
+    // columns above S 2^-5, above about S 2^-7, above S 2^-10: by the first two digits
+    uint32_t over[3], tile_over;
+    bool ask = false;
 #pragma unroll
     for (int d = 0; d < TMX_ND; ++d) {
         const float sc = tern_pow2(e - 5 * d);
         const u6v q = __builtin_bit_cast(u6v, __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(x.u, x.v, sc));
         put(d, q);
-        if (d == TMX_ND - 1 && __ballot(spread) == 0) break;
+        if (CHECK && d == 0) {
+            over[0] = tern_at_least<1>(q);
+            tile_over = many ? or_half(over[0]) : 0xFFFFFFFFu;
+        }
+        if (CHECK && d == 1) {
+            over[1] = over[0] | tern_at_least<4>(q);
+            over[2] = over[0] | tern_at_least<1>(q);
+            ask = mx != 0.0f && (__builtin_popcount(over[0]) <= 32 - 12 || __builtin_popcount(over[1]) <= 32 - 7 ||
+                                 __builtin_popcount(over[2]) <= 32 - 4 || tile_over != 0xFFFFFFFFu);
+        }
+        if (CHECK && d == TMX_ND - 1 && __ballot(ask) == 0) break;
         const f32v b = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(q, sc);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
@@ -81,14 +137,21 @@ __device__ __forceinline__ int tern_digits(TernBlock& x, bool& wide, const Put& 
             x.v[i] -= b[2 * i + 1];
         }
     }
-    wide = false;
-    if (spread) {
-        uint32_t rest = 0;
+    if constexpr (CHECK) {
+        wide = false;
+        if (__ballot(ask) != 0) {
+            // rare: of these columns, those whose digits do not end
+            uint32_t rest = 0;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) rest |= __float_as_uint(x.u[i]) | __float_as_uint(x.v[i]);
-        wide = (rest & 0x7FFFFFFFu) != 0;
+            for (int i = 0; i < 16; ++i) {
+                rest |= x.u[i] != 0.0f ? 1u << tern_bit(2 * i) : 0u;
+                rest |= x.v[i] != 0.0f ? 1u << tern_bit(2 * i + 1) : 0u;
+            }
+            wide = ask && (__builtin_popcount(rest & ~over[0]) >= 12 || __builtin_popcount(rest & ~over[1]) >= 7 ||
+                           __builtin_popcount(rest & ~over[2]) >= 4 || (rest & ~tile_over) != 0);
+        }
     }
-    return e;
+    return eb == 255 ? 255 : e;
 }
 // element e of the fragment order: its column in the 32
 __host__ __device__ constexpr int tern_mx_col(int e) { return 16 * (e >> 4) + 2 * (e & 7) + ((e >> 3) & 1); }
@@ -125,7 +188,7 @@ __device__ __forceinline__ void tmx_copy4(const void* g, const uint8_t* lds) {
 // x's digits: one block per 64 tokens and group; work: [tile][group] TMX_TILE bytes, then a flag word each. The rows
 // come through LDS (a copy moves 512 contiguous bytes of two tokens; a thread then takes 32 columns of one token):
 // read straight into registers, a wave would touch 64 lines per load. Tokens past T get zeros.
-__global__ __launch_bounds__(256) void tern_digits_kernel(const float* __restrict__ x, int64_t x_ts, int T, int K,
+__global__ __launch_bounds__(256, 4) void tern_digits_kernel(const float* __restrict__ x, int64_t x_ts, int T, int K,
                                                           uint8_t* __restrict__ work) {
     constexpr int PAIR = 1040;  // LDS pitch of two tokens' 512 bytes
     __shared__ __attribute__((aligned(16))) uint8_t rows[32 * PAIR];
@@ -152,8 +215,10 @@ __global__ __launch_bounds__(256) void tern_digits_kernel(const float* __restric
         for (int i = 0; i < 16; ++i) v.u[i] = v.v[i] = 0.0f;
     }
     bool wide;
-    const int e = tern_digits(v, wide, [&](int d, u6v q) { tern_mx_put(out, kh, d, m + 32 * h, q); });
+    const int e = tern_digits<true>(v, T - t0 - 32 * u >= 8, wide,
+                                    [&](int d, u6v q) { tern_mx_put(out, kh, d, m + 32 * h, q); });
     out[TMX_DIG + 4 * (m + 32 * h) + kh] = (uint8_t)e;
+    out[TMX_DIG + 4 * (m + 32 * h) + 2 + kh] = wide;
     __shared__ int wide_lds[4];
     const bool any = __ballot(wide) != 0;
     if (lane == 0) wide_lds[wave] = any;
@@ -259,24 +324,37 @@ __global__ __launch_bounds__(64 * W * KS, 2) void tern_mx_kernel(TernArgs a, int
         const float* p = a.x + (int64_t)min(xtok, a.T - 1) * a.x_ts + g * TMX_G + 64 * xh + 32 * xkh;
         tern_block_load(v, [&](int c) { return reinterpret_cast<const f4*>(p)[c]; });
     };
-    // the thread's 32 values as digits into a stage (second: their remainders' digits where they need them, else zeros);
-    // returns whether they need a second set
-    auto make_tiles = [&](TernBlock& v, uint8_t* sb, bool second) __attribute__((always_inline)) {
-        if (xtile >= MT) return false;
+    // the thread's 32 values as digits into a stage; returns whether they need a second set
+    auto make_tiles = [&](TernBlock& v, uint8_t* sb) __attribute__((always_inline)) {
+        bool wide = false;
+        if (xtile >= MT) return wide;
         uint8_t* dst = sb + xtile * TMX_TILE;
-        bool wide = false, drop = xtok >= a.T;
+        if (xtok >= a.T) {
+#pragma unroll
+            for (int c = 0; c < 16; ++c) v.u[c] = v.v[c] = 0.0f;
+        }
+        const int e = tern_digits<true>(v, a.T - t0 - 32 * xtile >= 8, wide,
+                                        [&](int d, u6v q) { tern_mx_put(dst, xkh, d, xm + 32 * xh, q); });
+        dst[TMX_DIG + 4 * (xm + 32 * xh) + xkh] = (uint8_t)e;
+        dst[TMX_DIG + 4 * (xm + 32 * xh) + 2 + xkh] = wide;
+        return wide;
+    };
+    // the remainders' digits in the tiles' place, zeros for blocks that need none
+    auto make_second = [&](TernBlock& v, uint8_t* sb) __attribute__((always_inline)) {
+        if (xtile >= MT) return;
+        uint8_t* dst = sb + xtile * TMX_TILE;
+        const bool drop = dst[TMX_DIG + 4 * (xm + 32 * xh) + 2 + xkh] == 0;
+        bool none;
         int e = 0;
 #pragma unroll 1
-        for (int pass = second ? 0 : 1; pass < 2; ++pass) {
+        for (int pass = 0; pass < 2; ++pass) {
+            e = tern_digits<false>(v, false, none, [&](int d, u6v q) { tern_mx_put(dst, xkh, d, xm + 32 * xh, q); });
             if (drop) {
 #pragma unroll
                 for (int c = 0; c < 16; ++c) v.u[c] = v.v[c] = 0.0f;
             }
-            e = tern_digits(v, wide, [&](int d, u6v q) { tern_mx_put(dst, xkh, d, xm + 32 * xh, q); });
-            drop = !wide;
         }
         dst[TMX_DIG + 4 * (xm + 32 * xh) + xkh] = (uint8_t)e;
-        return wide;
     };
     static_assert(128 * MT <= 64 * W, "a thread per 32 columns of a token");
 
@@ -349,7 +427,7 @@ __global__ __launch_bounds__(64 * W * KS, 2) void tern_mx_kernel(TernArgs a, int
         block_wide = __ballot(f != 0) != 0;
     }
     auto stage_tiles = [&](TernBlock& v, uint8_t* sb, int s) __attribute__((always_inline)) {
-        const bool any = __ballot(make_tiles(v, sb, false)) != 0;
+        const bool any = __ballot(make_tiles(v, sb)) != 0;
         if (lane == 0) wide_lds[s][wv] = any;
     };
     uint8_t* const st0 = lds0 + ks * STAGE;
@@ -400,7 +478,7 @@ __global__ __launch_bounds__(64 * W * KS, 2) void tern_mx_kernel(TernArgs a, int
             // rare: the remainders of the blocks that need them take the tiles' place
             __syncthreads();
             load_x(g, v);
-            make_tiles(v, sb, true);
+            make_second(v, sb);
             __syncthreads();
             if (KS == 1 || j < cnt) products(sb, sc);
         }

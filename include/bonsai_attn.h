@@ -361,10 +361,11 @@ bn_status bn_norm_rotate(bn_ctx* ctx, bn_stream stream, const bn_norm_args* a);
 bn_status bn_ternary_check(const bn_ternary_args* a);
 /* y = (add ? y : 0) + x W^T (+ LoRA) for each matrix (model.rs:455-596: qmm_multi / qmv4 for one token, qmvr,
  * qmvx and qmm3 for more; kernels.metal:431-500 qmm, 664-709 qmvxm). Results are fp32 sums of exact products up to
- * x's 2^-22 relative split error (T > 32: 2^-24 of the largest of 32 columns, the rest of a block that is far above
- * the others included; the reference computes in fp32), identical from call to call, for any finite x up to about
- * 4e9 in magnitude (x beyond fp16's range is scaled by a power of two inside the call). y must not overlap x, W or
- * another matrix's y. */
+ * x's split error (the reference computes in fp32), identical from call to call, for any finite x up to about 4e9 in
+ * magnitude (x beyond fp16's range is scaled by a power of two inside the call). The split error is 2^-22 of each value
+ * up to 32 tokens. Beyond, it is 2^-24 of the largest of 32 neighbouring columns of a token, and 2^-48 of it where 12 or
+ * more of the 32 lie 2^6 below that one, 7 or more 2^9, 4 or more 2^11, or a column lies 2^6 below it in all of the 8 to
+ * 32 tokens of a tile. y must not overlap x, W or another matrix's y. */
 bn_status bn_ternary_matmul(bn_ctx* ctx, bn_stream stream, const bn_ternary_args* a);
 /* Bytes of bn_ternary_args.work for T tokens of width k (0 when T <= 32: those calls use none). With a workspace the
  * call runs two kernels: x split into its digits once, then the GEMM streaming those tiles; without, every block of the

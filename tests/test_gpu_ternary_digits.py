@@ -1,8 +1,8 @@
 """bn_ternary_matmul with more than 32 tokens (bn_ternary_mx.h) against float64: x as five base-32 digits per block of 32
-columns of a token, with a second set where one value of a block is far above the rest.
+columns of a token, with a second set where columns of a block lie far below its largest.
 
-Bound per output, from the arithmetic: a block's digits end within 2^-24 of the power of two below its largest value
-(for a block with a second set: of its remainder's, so 2^-44), and each group's sum takes at most 20 additions of MFMA
+Bound per output, from the arithmetic: a block's digits end within 2^-24 of its largest value (where 12 or more columns
+lie 2^6 below that, it has a second set: 2^-24 of the remainder's, so 2^-44), and each group's sum takes at most 20 additions of MFMA
 results and one fma, each rounding the running sum by at most 2^-23 of sum |x w| (2^-24 for one rounding, doubled for an
 accumulation inside the MFMA); the groups' sums add one more each.
 """
@@ -37,7 +37,7 @@ def exact(w, s, codes, x):
     x = x.astype(np.float64)
     blocks = np.abs(x).reshape(x.shape[0], -1, 32)
     mx = blocks.max(-1)
-    cut = np.where(blocks.sum(-1) < 4 * mx, 2.0 ** -44, 2.0 ** -24) * mx
+    cut = np.where((blocks <= mx[..., None] / 64).sum(-1) >= 12, 2.0 ** -44, 2.0 ** -24) * mx
     aw = np.abs(full)
     split = cut @ aw.reshape(aw.shape[0], -1, 32).sum(-1).T
     groups = x.shape[1] // 128
@@ -84,3 +84,32 @@ def test_digits_nonfinite_token(gpu):
         assert np.isnan(got[[4, 66]]).all()
         rest = np.setdiff1d(np.arange(T), [4, 66])
         assert np.array_equal(got[rest], clean[rest])
+
+
+@pytest.mark.parametrize("large,mag", [(5, 1e3), (6, 1e4), (8, 30.0), (8, 2e4), (16, 300.0), (24, 1e3), (24, 1e5),
+                                       (28, 1e4), (31, 300.0), (31, 1e5)])
+def test_small_columns_beside_large_ones(gpu, large, mag):
+    """Some columns of every 32 (the same for all tokens, as channels of another scale are) hold values mag times the
+    others', under weights 0: what is left are the small columns' products, to workload.ternary_tolerance (2e-5 of their
+    norm) as for any other call. Then with the large values in one token of 16 only, 24 of 32 columns at most (its own
+    columns decide there). T = 72: the last tile has 8 tokens."""
+    torch, ctx, _ = gpu
+    T, K, O = 72, 768, 256
+    w, s, codes = workload.ternary_weights(0x7C00 + large, O, K, True)
+    rank = np.argsort(np.argsort(oracle.normal(0x7C00 + large, 2, (K // 32, 32)), axis=1), axis=1).reshape(-1)
+    big = rank < large
+    codes[:, big] = 1
+    w = workload.pack_codes(codes)
+    base = oracle.normal(0x7C00 + large, 1, (T, K)).copy()
+    for tokens in (np.arange(T), np.arange(3, T, 16)):
+        if len(tokens) < T and large > 24:
+            continue
+        print(f"ternary digits, {large} of 32 columns x {mag} in {len(tokens)} tokens", flush=True)
+        x = base.copy()
+        x[np.ix_(tokens, big)] *= np.float32(mag)
+        full = (codes.astype(np.float64) - 1) * np.repeat(oracle.f16_to_f32(s).astype(np.float64), 128, axis=1)
+        ref, tol = x.astype(np.float64) @ full.T, workload.ternary_tolerance(x, codes, s)
+        for work in (True, False):
+            got = call(torch, ctx, [(w, s, codes)], x, work)[0]
+            worst = float(np.max(np.abs(got - ref) / tol))
+            assert worst <= 1, f"workspace {work}: {worst:.2f} of the bound"
