@@ -914,32 +914,56 @@ bn_status run_ternary(bn_ctx* ctx, hipStream_t st, const bn_ternary_args* a) {
     //  - 32 x 256 up to two per CU (their two stages let three stay on a CU; 4B o_proj of 1,017 tokens: 64.4 against
     //    74.4 with 64 x 256, of 2,000: 114 against 104)
     //  - 64 x 256 beyond: each decoded weight feeds twice the MFMAs
-    // Without a workspace every block makes its own digits, vector work that twice the rows halve: 64 x 512 where such
-    // blocks fill their rounds over the CUs (4B q/k/v of 4,096 tokens: 387 against 410; of 1,017: 151 against 133).
     const int64_t dig_blocks = ceil_div(a->T, 64) * (int64_t)(a->k / bn::TMX_G);
     const int64_t small = ceil_div(a->T, 32) * ceil_div(rows, 128), mid = ceil_div(a->T, 32) * ceil_div(rows, 256);
     const int64_t large = ceil_div(a->T, 64) * ceil_div(rows, 256);
-    const int64_t cus = ctx->cus, large8 = ceil_div(a->T, 64) * ceil_div(rows, 512);
+    const int64_t cus = ctx->cus;
     const bool split = 2 * small <= 3 * cus;
     if (large > INT32_MAX) return set_err(ctx->err, BN_EINVAL, "T * rows too large for one launch");
     const uint8_t* work = static_cast<const uint8_t*>(a->work);
-    const int rt128 = (int)ceil_div(rows, 128), rt256 = (int)ceil_div(rows, 256);
+    const int rt128 = (int)ceil_div(rows, 128), rt256 = (int)ceil_div(rows, 256), rt512 = (int)ceil_div(rows, 512);
     if (work && dig_blocks <= INT32_MAX) {
         bn_launch(ctx, bn::tern_digits_kernel, dim3((unsigned)dig_blocks), dim3(256), 0, st, a->x, a->x_ts, (int)a->T,
                   (int)a->k, static_cast<uint8_t*>(a->work));
         if (split)
-            bn_launch(ctx, (bn::tern_mx_kernel<2, 1, 2, true>), dim3((unsigned)small), dim3(256), 0, st, t, rt128, work);
+            bn_launch(ctx, (bn::tern_mx_kernel<2, 1, 2, 0>), dim3((unsigned)small), dim3(256), 0, st, t, rt128, work);
         else if (mid <= 2 * cus)
-            bn_launch(ctx, (bn::tern_mx_kernel<4, 1, 1, true>), dim3((unsigned)mid), dim3(256), 0, st, t, rt256, work);
+            bn_launch(ctx, (bn::tern_mx_kernel<4, 1, 1, 0>), dim3((unsigned)mid), dim3(256), 0, st, t, rt256, work);
         else
-            bn_launch(ctx, (bn::tern_mx_kernel<4, 2, 1, true>), dim3((unsigned)large), dim3(256), 0, st, t, rt256, work);
-    } else if (split) {
-        bn_launch(ctx, (bn::tern_mx_kernel<2, 1, 2, false>), dim3((unsigned)small), dim3(256), 0, st, t, rt128, work);
-    } else if (8 * large8 >= 6 * cus * ceil_div(large8, cus)) {
-        bn_launch(ctx, (bn::tern_mx_kernel<8, 2, 1, false>), dim3((unsigned)large8), dim3(512), 0, st, t,
-                  (int)ceil_div(rows, 512), work);
+            bn_launch(ctx, (bn::tern_mx_kernel<4, 2, 1, 0>), dim3((unsigned)large), dim3(256), 0, st, t, rt256, work);
+        return launched(ctx, "tern_mx_kernel");
+    }
+    // Without a workspace every block makes its own digits, vector work that many rows share: 512 of them, but for the
+    // smallest calls. One such block stays on a CU, so a call takes rounds of 64-token blocks, or of 32-token blocks at
+    // 0.65 of their time (4B q/k/v: 70 against 45 us, 4B o_proj 121 against 76), or of both: full rounds of the first
+    // and one of the second for the tokens left, in a launch of its own (4B o_proj of 4,096 tokens: 202 us against 239
+    // and 222; 4B q/k/v of 1,017: 121 against 137 and 130).
+    if (split) {
+        bn_launch(ctx, (bn::tern_mx_kernel<2, 1, 2, 2>), dim3((unsigned)small), dim3(256), 0, st, t, rt128, work);
+        return launched(ctx, "tern_mx_kernel");
+    }
+    auto tokens = [&](int64_t from, int64_t n, bool tiles64) {
+        bn::TernArgs p = t;
+        for (bn::TernMat& m : p.m) m.y += from * m.y_ts;
+        p.x += from * p.x_ts;
+        if (p.lu) p.lu += from * p.lu_ts;
+        p.T = (int)n;
+        const dim3 grid((unsigned)(ceil_div(n, tiles64 ? 64 : 32) * rt512));
+        if (tiles64)
+            bn_launch(ctx, (bn::tern_mx_kernel<8, 2, 1, 3>), grid, dim3(512), 0, st, p, rt512, work);
+        else
+            bn_launch(ctx, (bn::tern_mx_kernel<8, 1, 1, 3>), grid, dim3(512), 0, st, p, rt512, work);
+    };
+    const int64_t T = a->T;
+    auto rounds = [&](int64_t n, int64_t tile) { return ceil_div(ceil_div(n, tile) * rt512, cus); };
+    const int64_t r64 = rounds(T, 64), full = 64 * ((r64 - 1) * cus / rt512);  // tokens of the full rounds
+    const double c64 = (double)r64, c32 = 0.65 * rounds(T, 32);
+    const double c_both = full > 0 ? r64 - 1 + 0.65 * rounds(T - full, 32) : 1e30;
+    if (c_both < c64 && c_both < c32) {
+        tokens(0, full, true);
+        tokens(full, T - full, false);
     } else {
-        bn_launch(ctx, (bn::tern_mx_kernel<4, 2, 1, false>), dim3((unsigned)large), dim3(256), 0, st, t, rt256, work);
+        tokens(0, T, c64 <= c32);
     }
     return launched(ctx, "tern_mx_kernel");
 }

@@ -74,6 +74,17 @@ __device__ __forceinline__ int call_off(const uint32_t* dyn, int off_max) {
     return off_max;
 }
 
+typedef __attribute__((address_space(3))) void pf_lds_void_t;
+// 16 bytes per lane from global memory into LDS at lds_base + 16 lane (global_load_lds_dwordx4), written as
+// assembly so that the compiler does not track it: its own tracking of these copies cannot tell the stages (or the
+// K and V halves) of one LDS array apart and would wait for every copy in flight before each operand read. The
+// caller orders the copies against the reads itself (s_waitcnt vmcnt, then a wave or block barrier). M0 carries the
+// LDS base; nothing else in the kernels that use this sets M0.
+__device__ __forceinline__ void pf_copy16(const void* g, const uint8_t* lds_base) {
+    const uint32_t la = (uint32_t)(uintptr_t)(pf_lds_void_t*)lds_base;
+    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(la) : "memory");
+}
+
 // Wave-local LDS hand-off: the wave's LDS writes are complete and visible to its own lanes afterwards.
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

@@ -74,23 +74,12 @@ __host__ __device__ inline int pf_splits(int nt, int ct) { return (nt + ct - 1) 
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef short pf_s4v __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) pf_s4v pf_lds_s4_t;
-typedef __attribute__((address_space(3))) void pf_lds_void_t;
 
 __device__ __forceinline__ h8 pf_lds_h8(const uint8_t* p) { return *reinterpret_cast<const h8*>(p); }
 __device__ __forceinline__ h4 pf_lds_tr(const uint8_t* p) {
     return __builtin_bit_cast(h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((pf_lds_s4_t*)(p)));
 }
 __device__ __forceinline__ void pf_wait_vm0() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
-// 16 bytes per lane from global memory into LDS at lds_base + 16 lane (global_load_lds_dwordx4), written as
-// assembly so that the compiler does not track it: its own tracking of these copies cannot tell the stages (or the
-// K and V halves) of one LDS array apart and would wait for every copy in flight before each operand read. The
-// caller orders the copies against the reads itself (s_waitcnt vmcnt, then a wave or block barrier). M0 carries the
-// LDS base; nothing else in the kernels that use this sets M0.
-__device__ __forceinline__ void pf_copy16(const void* g, const uint8_t* lds_base) {
-    const uint32_t la = (uint32_t)(uintptr_t)(pf_lds_void_t*)lds_base;
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(la) : "memory");
-}
 
 __global__ __launch_bounds__(512) void prefill_kernel(PrefillArgs a) {
     // stage 0 and stage 1 of both groups are separate LDS objects: the compiler then sees that a tile copy into

@@ -16,14 +16,13 @@
 // which a row whose weights are 0 on the large columns shows. Such a block's remainder is written as five more digits and
 // multiplied by a second pass over the group (flagged per 32-token tile; blocks that need none are zero there). It is
 // made where the digits of these columns do not end:
-//   - at least 12 of the block's columns within S 2^-5, 7 within S 2^-7 or 4 within S 2^-10; or
+//   - at least 12 of the block's columns within S 2^-5, or 6 within S 2^-7.7; or
 //   - a column within S 2^-5 in every token of the tile (of 8 tokens or more), as columns of another scale are.
-// With small columns in the same places for a tile's tokens their error is then at most 1e-6 of their norm, and 2.2e-6
+// With small columns in the same places for a tile's tokens their error is then at most 1e-6 of their norm, and 2.3e-6
 // for single tokens with up to 25 large columns of 32 (worst of 1 to 31 large columns, 8 to 10^5 times the others, weights
 // 0 under them; the digits alone: 3e-3). The rules are no wider because a step with a second pass takes more than
-// twice as long, and the blocks of a call that runs in one round wait for it: they take 2e-7 of the blocks of normally
-// distributed values for such (with 6 and 3 in the places of 7 and 4 it was 2e-5, and calls of 1,000 to 2,000 tokens
-// took 10-20% longer). The block scale covers fp32's exponents; a block with an infinity or a NaN gets the scale NaN,
+// twice as long, and the blocks of a call that runs in one round wait for it: they take 1e-7 of the blocks of normally
+// distributed values for such (with 2e-5 of them calls of 1,000 to 2,000 tokens took 10-20% longer). The block scale covers fp32's exponents; a block with an infinity or a NaN gets the scale NaN,
 // and the token's outputs are NaN.
 // Measured (MI355X, the 4B q/k/v projections of 4,096 tokens): 303 us (digits 17, GEMM 285) against 368 for the fp16
 // hi/lo split, whose 1.16 PFLOP/s of products were the rate of a large library product here; error against 64-bit sums
@@ -36,8 +35,9 @@
 // 16 (e / 8 / 2) + 2 (e % 8) + (e / 8) % 2: a word's even codes, then its odd ones, as the decode leaves them.
 //
 // tern_digits_kernel writes x's digits once per call as the tiles the GEMM reads (15 KB per 32 tokens and group);
-// tern_mx_kernel<W, MT, KS, PRE> multiplies: PRE = true copies those tiles into LDS, false (no workspace) makes the
-// same digits from x itself. Both run the same products in the same order: identical results.
+// tern_mx_kernel<W, MT, KS, NS> multiplies: NS = 0 copies those tiles into LDS, NS = 2 or 3 (no workspace) brings x itself
+// into as many stages of LDS and makes the same digits there. All run the same products in the same order: identical
+// results.
 #pragma once
 #include "bn_ternary.h"
 
@@ -111,8 +111,8 @@ __device__ __forceinline__ int tern_digits(TernBlock& x, bool many, bool& wide, 
     for (int i = 0; i < 16; ++i) asm("v_maximum3_f32 %0, |%1|, |%2|, %0" : "+v"(mx) : "v"(x.u[i]), "v"(x.v[i]));
     const int eb = (__float_as_int(mx) >> 23) & 255;
     const int e = max(eb - 1, 28);  // 28: the last digit's scale stays normal
-    // columns above S 2^-5, above about S 2^-7, above S 2^-10: by the first two digits
-    uint32_t over[3], tile_over;
+    // columns above S 2^-5, above S 2^-7.7: by the first two digits
+    uint32_t over[2], tile_over;
     bool ask = false;
 #pragma unroll
     for (int d = 0; d < TMX_ND; ++d) {
@@ -124,10 +124,9 @@ __device__ __forceinline__ int tern_digits(TernBlock& x, bool many, bool& wide, 
             tile_over = many ? or_half(over[0]) : 0xFFFFFFFFu;
         }
         if (CHECK && d == 1) {
-            over[1] = over[0] | tern_at_least<4>(q);
-            over[2] = over[0] | tern_at_least<1>(q);
-            ask = mx != 0.0f && (__builtin_popcount(over[0]) <= 32 - 12 || __builtin_popcount(over[1]) <= 32 - 7 ||
-                                 __builtin_popcount(over[2]) <= 32 - 4 || tile_over != 0xFFFFFFFFu);
+            over[1] = over[0] | tern_at_least<3>(q);
+            ask = mx != 0.0f && (__builtin_popcount(over[0]) <= 32 - 12 || __builtin_popcount(over[1]) <= 32 - 6 ||
+                                 tile_over != 0xFFFFFFFFu);
         }
         if (CHECK && d == TMX_ND - 1 && __ballot(ask) == 0) break;
         const f32v b = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(q, sc);
@@ -147,8 +146,8 @@ __device__ __forceinline__ int tern_digits(TernBlock& x, bool many, bool& wide, 
                 rest |= x.u[i] != 0.0f ? 1u << tern_bit(2 * i) : 0u;
                 rest |= x.v[i] != 0.0f ? 1u << tern_bit(2 * i + 1) : 0u;
             }
-            wide = ask && (__builtin_popcount(rest & ~over[0]) >= 12 || __builtin_popcount(rest & ~over[1]) >= 7 ||
-                           __builtin_popcount(rest & ~over[2]) >= 4 || (rest & ~tile_over) != 0);
+            wide = ask && (__builtin_popcount(rest & ~over[0]) >= 12 || __builtin_popcount(rest & ~over[1]) >= 6 ||
+                           (rest & ~tile_over) != 0);
         }
     }
     return eb == 255 ? 255 : e;
@@ -169,12 +168,22 @@ __device__ __forceinline__ void tern_block_load(TernBlock& x, const Ld& ld) {
     }
 }
 // digit d's six words of (lane, kh) into a tile at p (global memory or LDS): words 6 kh .. of the lane's 12, four of
-// them in each 1 KB plane, so that a lane reads both halves' operands in three 16-byte reads
+// them in each 1 KB plane, so that a lane reads both halves' operands in three 16-byte reads. kh: the same for a wave
+// (the words are selected by a branch, not by six selects).
 __device__ __forceinline__ void tern_mx_put(uint8_t* p, int kh, int d, int lane, u6v q) {
     uint8_t* f = p + d * TMX_FRAG + 16 * lane;
-    *reinterpret_cast<u4*>(f + (kh ? 2048 : 0)) = kh ? u4{q[2], q[3], q[4], q[5]} : u4{q[0], q[1], q[2], q[3]};
-    *reinterpret_cast<u2*>(f + 1024 + 8 * kh) = kh ? u2{q[0], q[1]} : u2{q[4], q[5]};
+    if (kh) {
+        *reinterpret_cast<u2*>(f + 1024 + 8) = u2{q[0], q[1]};
+        *reinterpret_cast<u4*>(f + 2048) = u4{q[2], q[3], q[4], q[5]};
+    } else {
+        *reinterpret_cast<u4*>(f) = u4{q[0], q[1], q[2], q[3]};
+        *reinterpret_cast<u2*>(f + 1024) = u2{q[4], q[5]};
+    }
 }
+// A tile made in its block's LDS: 8 KB per kh, which hold the 64 columns of x (32 tokens) that the digits come from until
+// the wave has read them. Per digit words 0..3 of a lane, then words 4, 5; the blocks' scale bytes; whether each is wide;
+// a word, whether any is.
+constexpr int TMX_RAW = 8192, TMX_RDIG = 64 * 24, TMX_RSCALE = TMX_ND * TMX_RDIG, TMX_RANY = TMX_RSCALE + 128;
 
 typedef __attribute__((address_space(3))) void tmx_lds_t;
 // 16 (4) bytes per lane from global memory into LDS at lds + 16 lane (4 lane)
@@ -203,8 +212,8 @@ __global__ __launch_bounds__(256, 4) void tern_digits_kernel(const float* __rest
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    // wave: tile wave / 2, lane half h = wave % 2 of its fragments; lane: token lane % 32, half kh = lane / 32
-    const int u = wave >> 1, h = wave & 1, m = lane & 31, kh = lane >> 5, b = 2 * h + kh;
+    // wave: tile wave / 2, MFMA half kh = wave % 2; lane: token lane % 32, lane half h = lane / 32 of its fragments
+    const int u = wave >> 1, kh = wave & 1, m = lane & 31, b = 2 * (lane >> 5) + kh;
     const int tile = 2 * tt + u;
     uint8_t* out = work + ((size_t)tile * ng + g) * TMX_TILE;
     TernBlock v;
@@ -216,9 +225,9 @@ __global__ __launch_bounds__(256, 4) void tern_digits_kernel(const float* __rest
     }
     bool wide;
     const int e = tern_digits<true>(v, T - t0 - 32 * u >= 8, wide,
-                                    [&](int d, u6v q) { tern_mx_put(out, kh, d, m + 32 * h, q); });
-    out[TMX_DIG + 4 * (m + 32 * h) + kh] = (uint8_t)e;
-    out[TMX_DIG + 4 * (m + 32 * h) + 2 + kh] = wide;
+                                    [&](int d, u6v q) { tern_mx_put(out, kh, d, lane, q); });
+    out[TMX_DIG + 4 * lane + kh] = (uint8_t)e;
+    out[TMX_DIG + 4 * lane + 2 + kh] = wide;
     __shared__ int wide_lds[4];
     const bool any = __ballot(wide) != 0;
     if (lane == 0) wide_lds[wave] = any;
@@ -239,25 +248,28 @@ __device__ __forceinline__ void tern_fp4(uint32_t w, int& even, int& odd) {
     odd = (int)((n & 0xCCCCCCCCu) | ((q >> 1) & ~0xCCCCCCCCu));
 }
 
-// stage bytes of a wave group: its MT x tiles, then the waves' codes (64 rows x 32 bytes each)
-__host__ __device__ constexpr int tmx_stage(int W, int MT) { return MT * TMX_TILE + W * 2048; }
 // copies of fragments per wave and group of columns (1 KB each, the last repeated where they do not divide)
 __host__ __device__ constexpr int tmx_frag_copies(int W, int MT) { return (15 * MT + W - 1) / W; }
 
 // KS wave groups of W waves x 64 rows, 32 MT tokens; the groups split the columns and add their sums at the end, in
-// order. PRE: x's digits come from tern_digits_kernel's tiles, otherwise from x. Per 128 columns a wave multiplies MT
-// token tiles x 2 row tiles x 2 halves x 5 digits (32 cycles each) into a fresh accumulator per tile pair, which one
-// fma per output adds, times the row scale, to the running sums. Two stages in LDS, the next step's copies in flight
-// during a step's products; one barrier per step.
-template <int W, int MT, int KS, bool PRE>
+// order. Per 128 columns a wave multiplies MT token tiles x 2 row tiles x 2 halves x 5 digits (32 cycles each) into a
+// fresh accumulator per tile pair, which one fma per output adds, times the row scale, to the running sums. One barrier
+// per step. NS = 0 (PRE): x's digits come from tern_digits_kernel's tiles; two stages in LDS, the next step's copies in
+// flight during a step's products. NS = 2: x comes instead, and the next step's digits are made from it after the products.
+// NS = 3: x comes two steps ahead, and with twice the waves that a stage's tiles take, half of the waves make the next
+// step's digits while the others multiply, turn about (8 waves x 64 rows, 4B q/k/v of 4,096 tokens: 355 us; with two
+// stages 371, and 392 with x read by token and block, where each load touches 64 places; the copies' addresses and the
+// digits are vector work, two thirds of a step's as long as 256 rows share it).
+template <int W, int MT, int KS, int NS>
 __global__ __launch_bounds__(64 * W * KS, 2) void tern_mx_kernel(TernArgs a, int row_tiles,
                                                                  const uint8_t* __restrict__ work) {
+    constexpr bool PRE = NS == 0;
     static_assert(MT == 1 || MT == 2, "token tiles per block (x's tiles come in pairs)");
-    constexpr int BM = 32 * MT, STAGE = tmx_stage(W, MT), ST_W = MT * TMX_TILE;
-    // separate arrays, so that the compiler can tell one stage's copies from another's reads
-    __shared__ __attribute__((aligned(1024))) uint8_t lds0[KS * STAGE];
-    __shared__ __attribute__((aligned(1024))) uint8_t lds1[KS * STAGE];
-    __shared__ int wide_lds[2][W * KS];
+    // a stage of a wave group: its MT x tiles, then the waves' codes (64 rows x 32 bytes each)
+    constexpr int TILE = PRE ? TMX_TILE : 2 * TMX_RAW, BM = 32 * MT, ST_W = MT * TILE, STAGE = ST_W + W * 2048;
+    // separate arrays, so that the compiler can tell one stage's copies from another's reads (PRE = false: pf_copy16's)
+    __shared__ __attribute__((aligned(1024))) uint8_t lds0[(PRE ? 1 : NS) * KS * STAGE];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds1[PRE ? KS * STAGE : 1];
     static_assert(KS == 1 || (KS - 1) * W * MT * 8192 <= KS * STAGE, "the groups' sums fit a stage");
     const int lane = (int)threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), ks = wv / W, wave = wv % W;
@@ -302,10 +314,29 @@ __global__ __launch_bounds__(64 * W * KS, 2) void tern_mx_kernel(TernArgs a, int
                 sw[nt] = *p;
         }
     };
-    // the copies of column group g into a stage
-    auto issue = [&](int g, const uint8_t* sb) __attribute__((always_inline)) {
+    // PRE = false: the waves that make a stage's tiles, a wave per tile and kh; with waves to spare, others for each stage
+    // (mk: the wave's tile and kh). A maker copies 32 tokens x 64 columns in pieces of 128 contiguous bytes (read by token
+    // and block, each load would touch 64 places), copy i rows 4 i + lane / 16; a row's 16-byte chunks are swapped by its
+    // number, so that 16 tokens' reads below fall on distinct banks: four addresses per lane serve the 8 copies. Rows past
+    // T read the lane's first row, if that is past T the last.
+    constexpr int MK = 2 * MT, MK_S = 2 * MK <= W ? 2 : 1;
+    const int mk = wave % MK, tx = t0 + 32 * (mk >> 1);
+    auto makes = [&](int s) { return wave / MK == s % MK_S; };
+    const uint8_t* xp[PRE ? 1 : 4];
+    if constexpr (!PRE) {
+        const int q = lane >> 4, c = (lane & 15) ^ q;
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt) tmx_copy16(wsrc + nt * wtile + 32 * g, sb + ST_W + wave * 2048 + nt * 1024);
+        for (int k = 0; k < 4; ++k)
+            xp[k] = reinterpret_cast<const uint8_t*>(a.x + (int64_t)min(tx + q, a.T - 1) * a.x_ts + 32 * (mk & 1)) +
+                    ((256 * (c >> 3) + 16 * (c & 7)) ^ (64 * (k & 1)) ^ (256 * (k >> 1)));
+    }
+    // the copies of column group g into a stage (s: its number)
+    auto issue = [&](int g, const uint8_t* sb, int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+            if constexpr (PRE) tmx_copy16(wsrc + nt * wtile + 32 * g, sb + ST_W + wave * 2048 + nt * 1024);
+            else pf_copy16(wsrc + nt * wtile + 32 * g, sb + ST_W + wave * 2048 + nt * 1024);
+        }
         if constexpr (PRE) {
             constexpr int C = tmx_frag_copies(W, MT);
 #pragma unroll
@@ -315,48 +346,73 @@ __global__ __launch_bounds__(64 * W * KS, 2) void tern_mx_kernel(TernArgs a, int
             }
             const int u = wave & (MT - 1);
             tmx_copy4(tiles + u * tile_row + (size_t)g * TMX_TILE + TMX_DIG + 4 * lane, sb + u * TMX_TILE + TMX_DIG);
+        } else if (makes(s)) {
+            const int64_t gb = (int64_t)g * TMX_G * 4, row4 = a.x_ts * 16;
+            if (tx + 32 <= a.T) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) pf_copy16(xp[i & 3] + (gb + i * row4), sb + mk * TMX_RAW + i * 1024);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    pf_copy16(xp[i & 3] + gb + (tx + 4 * i + (lane >> 4) < a.T ? i * row4 : 0), sb + mk * TMX_RAW + i * 1024);
+            }
         }
     };
-    // x itself, for PRE = false and the second passes. Thread u of the wave group -> tile, token, 32 columns.
-    const int u_ = (int)threadIdx.x - 64 * W * ks;
-    const int xtile = u_ >> 7, xh = (u_ >> 6) & 1, xkh = (u_ >> 5) & 1, xm = u_ & 31, xtok = t0 + 32 * xtile + xm;
-    auto load_x = [&](int g, TernBlock& v) __attribute__((always_inline)) {
-        const float* p = a.x + (int64_t)min(xtok, a.T - 1) * a.x_ts + g * TMX_G + 64 * xh + 32 * xkh;
-        tern_block_load(v, [&](int c) { return reinterpret_cast<const f4*>(p)[c]; });
-    };
-    // the thread's 32 values as digits into a stage; returns whether they need a second set
-    auto make_tiles = [&](TernBlock& v, uint8_t* sb) __attribute__((always_inline)) {
-        bool wide = false;
-        if (xtile >= MT) return wide;
-        uint8_t* dst = sb + xtile * TMX_TILE;
-        if (xtok >= a.T) {
+    // PRE = false: a maker's columns of x, copied into a stage, as digits in their place (each lane's reads come before the
+    // wave's first write)
+    auto make_tiles = [&](uint8_t* sb, int s) __attribute__((always_inline)) {
+        if (!makes(s)) return;
+        if (NS == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        uint8_t* dst = sb + mk * TMX_RAW;
+        const int xm = lane & 31;
+        TernBlock v;
+        tern_block_load(v, [&](int c) {
+            return *reinterpret_cast<const f4*>(dst + 256 * xm + 16 * ((8 * (lane >> 5) + c) ^ (xm & 15)));
+        });
+        if (tx + xm >= a.T) {
 #pragma unroll
             for (int c = 0; c < 16; ++c) v.u[c] = v.v[c] = 0.0f;
         }
-        const int e = tern_digits<true>(v, a.T - t0 - 32 * xtile >= 8, wide,
-                                        [&](int d, u6v q) { tern_mx_put(dst, xkh, d, xm + 32 * xh, q); });
-        dst[TMX_DIG + 4 * (xm + 32 * xh) + xkh] = (uint8_t)e;
-        dst[TMX_DIG + 4 * (xm + 32 * xh) + 2 + xkh] = wide;
-        return wide;
+        bool wide;
+        const int e = tern_digits<true>(v, a.T - tx >= 8, wide, [&](int d, u6v q) {
+            *reinterpret_cast<u4*>(dst + d * TMX_RDIG + 16 * lane) = u4{q[0], q[1], q[2], q[3]};
+            *reinterpret_cast<u2*>(dst + d * TMX_RDIG + 1024 + 8 * lane) = u2{q[4], q[5]};
+        });
+        dst[TMX_RSCALE + lane] = (uint8_t)e;
+        dst[TMX_RSCALE + 64 + lane] = wide;
+        const bool any = __ballot(wide) != 0;
+        if (lane == 0) *reinterpret_cast<int*>(dst + TMX_RANY) = any;
     };
-    // the remainders' digits in the tiles' place, zeros for blocks that need none
-    auto make_second = [&](TernBlock& v, uint8_t* sb) __attribute__((always_inline)) {
-        if (xtile >= MT) return;
-        uint8_t* dst = sb + xtile * TMX_TILE;
-        const bool drop = dst[TMX_DIG + 4 * (xm + 32 * xh) + 2 + xkh] == 0;
+    // the second pass: the remainders' digits in the tiles' place, zeros for blocks that need none
+    auto make_second = [&](int g, uint8_t* sb) __attribute__((always_inline)) {
+        if (wave >= MK) return;
+        const int kh = wave & 1, xm = lane & 31, xtok = t0 + 32 * (wave >> 1) + xm;
+        TernBlock v;
+        const float* p = a.x + (int64_t)min(xtok, a.T - 1) * a.x_ts + g * TMX_G + 64 * (lane >> 5) + 32 * kh;
+        tern_block_load(v, [&](int c) { return reinterpret_cast<const f4*>(p)[c]; });
+        uint8_t* dst = PRE ? sb + (wave >> 1) * TMX_TILE : sb + wave * TMX_RAW;
+        uint8_t* sp = PRE ? dst + TMX_DIG + 4 * lane + kh : dst + TMX_RSCALE + lane;
+        const bool drop = sp[PRE ? 2 : 64] == 0;
         bool none;
         int e = 0;
 #pragma unroll 1
         for (int pass = 0; pass < 2; ++pass) {
-            e = tern_digits<false>(v, false, none, [&](int d, u6v q) { tern_mx_put(dst, xkh, d, xm + 32 * xh, q); });
+            e = tern_digits<false>(v, false, none, [&](int d, u6v q) {
+                if constexpr (PRE) {
+                    tern_mx_put(dst, kh, d, lane, q);
+                } else {
+                    *reinterpret_cast<u4*>(dst + d * TMX_RDIG + 16 * lane) = u4{q[0], q[1], q[2], q[3]};
+                    *reinterpret_cast<u2*>(dst + d * TMX_RDIG + 1024 + 8 * lane) = u2{q[4], q[5]};
+                }
+            });
             if (drop) {
 #pragma unroll
                 for (int c = 0; c < 16; ++c) v.u[c] = v.v[c] = 0.0f;
             }
         }
-        dst[TMX_DIG + 4 * (xm + 32 * xh) + xkh] = (uint8_t)e;
+        *sp = (uint8_t)e;
     };
-    static_assert(128 * MT <= 64 * W, "a thread per 32 columns of a token");
+    static_assert(MK <= W, "a thread per 32 columns of a token");
 
     f16x acc[MT][2];
 #pragma unroll
@@ -384,8 +440,14 @@ __global__ __launch_bounds__(64 * W * KS, 2) void tern_mx_kernel(TernArgs a, int
         }
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
-            const uint8_t* xl = sb + i * TMX_TILE;
-            const int ex = *reinterpret_cast<const int*>(xl + TMX_DIG + 4 * lane);
+            const uint8_t* xl = sb + i * TILE;
+            int ex, ex1;  // the blocks' scales: bytes 0 and 1 of ex, or byte 0 of each
+            if constexpr (PRE) {
+                ex = *reinterpret_cast<const int*>(xl + TMX_DIG + 4 * lane);
+            } else {
+                ex = xl[TMX_RSCALE + lane];
+                ex1 = xl[TMX_RAW + TMX_RSCALE + lane];
+            }
             f16x t[2];
 #pragma unroll
             for (int nt = 0; nt < 2; ++nt)
@@ -393,16 +455,27 @@ __global__ __launch_bounds__(64 * W * KS, 2) void tern_mx_kernel(TernArgs a, int
                 for (int e = 0; e < 16; ++e) t[nt][e] = 0.0f;
 #pragma unroll
             for (int d = TMX_ND - 1; d >= 0; --d) {
-                const u4* f = reinterpret_cast<const u4*>(xl + d * TMX_FRAG + 16 * lane);
-                const u4 w0 = f[0], w1 = f[64], w2 = f[128];
-                const i8v x0 = {(int)w0[0], (int)w0[1], (int)w0[2], (int)w0[3], (int)w1[0], (int)w1[1], 0, 0};
-                const i8v x1 = {(int)w1[2], (int)w1[3], (int)w2[0], (int)w2[1], (int)w2[2], (int)w2[3], 0, 0};
+                i8v x0, x1;
+                if constexpr (PRE) {
+                    const u4* f = reinterpret_cast<const u4*>(xl + d * TMX_FRAG + 16 * lane);
+                    const u4 w0 = f[0], w1 = f[64], w2 = f[128];
+                    x0 = i8v{(int)w0[0], (int)w0[1], (int)w0[2], (int)w0[3], (int)w1[0], (int)w1[1], 0, 0};
+                    x1 = i8v{(int)w1[2], (int)w1[3], (int)w2[0], (int)w2[1], (int)w2[2], (int)w2[3], 0, 0};
+                } else {
+                    auto half = [&](const uint8_t* f) {
+                        const u4 w0 = *reinterpret_cast<const u4*>(f + 16 * lane);
+                        const u2 w1 = *reinterpret_cast<const u2*>(f + 1024 + 8 * lane);
+                        return i8v{(int)w0[0], (int)w0[1], (int)w0[2], (int)w0[3], (int)w1[0], (int)w1[1], 0, 0};
+                    };
+                    x0 = half(xl + d * TMX_RDIG);
+                    x1 = half(xl + TMX_RAW + d * TMX_RDIG);
+                }
                 // the scale operands' byte selects are immediates: one call per digit
 #define TMX_MFMA(DD, SW)                                                                                        \
     for (int nt = 0; nt < 2; ++nt)                                                                              \
         t[nt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x0, b[nt][0], t[nt], 2, 4, 0, ex, DD, SW);      \
     for (int nt = 0; nt < 2; ++nt)                                                                              \
-        t[nt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x1, b[nt][1], t[nt], 2, 4, 1, ex, DD, SW)
+        t[nt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x1, b[nt][1], t[nt], 2, 4, PRE ? 1 : 0, PRE ? ex : ex1, DD, SW)
                 if (d == 4) { TMX_MFMA(0, sw1); }
                 if (d == 3) { TMX_MFMA(3, sw0); }
                 if (d == 2) { TMX_MFMA(2, sw0); }
@@ -426,22 +499,10 @@ __global__ __launch_bounds__(64 * W * KS, 2) void tern_mx_kernel(TernArgs a, int
             for (int u = 0; u < MT; ++u) f |= flags[(size_t)u * ng + g];
         block_wide = __ballot(f != 0) != 0;
     }
-    auto stage_tiles = [&](TernBlock& v, uint8_t* sb, int s) __attribute__((always_inline)) {
-        const bool any = __ballot(make_tiles(v, sb)) != 0;
-        if (lane == 0) wide_lds[s][wv] = any;
-    };
-    uint8_t* const st0 = lds0 + ks * STAGE;
-    uint8_t* const st1 = lds1 + ks * STAGE;
     load_s(group(0));
-    issue(group(0), st0);
-    if constexpr (!PRE) {
-        TernBlock v;
-        load_x(group(0), v);
-        stage_tiles(v, st0, 0);
-    }
-
-    // step j from stage sb (s: its number) while step j + 1 is brought into nb
-    auto step = [&](int j, uint8_t* sb, uint8_t* nb, int s) __attribute__((always_inline)) {
+    // step j from stage sb while a later step is brought into nb (PRE: the next; in place: the next of NS = 2 stages, the
+    // one after of 3, whose x the next step's digits are made from before the products)
+    auto step = [&](int j, uint8_t* sb, uint8_t* mb, uint8_t* nb) __attribute__((always_inline)) {
         // this step's copies of every wave have landed, and every wave is done with nb
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         const int g = group(j), gn = group(j + 1);
@@ -463,29 +524,56 @@ __global__ __launch_bounds__(64 * W * KS, 2) void tern_mx_kernel(TernArgs a, int
                 }
             }
         } else {
+            const uint8_t* sb0 = sb - ks * STAGE;
 #pragma unroll
-            for (int w = 0; w < W * KS; ++w) wide |= wide_lds[s][w] != 0;
+            for (int q = 0; q < KS; ++q)
+#pragma unroll
+                for (int k = 0; k < MK; ++k)
+                    wide |= *reinterpret_cast<const int*>(sb0 + q * STAGE + k * TMX_RAW + TMX_RANY) != 0;
+            wide = __builtin_amdgcn_readfirstlane(wide);
         }
-        issue(gn, nb);
-        TernBlock v;  // PRE = false: the next step's x, in flight during the products
-        if constexpr (!PRE) load_x(gn, v);
+        if constexpr (PRE || NS == 2) issue(gn, nb, j + 1);
+        else issue(group(j + 2), nb, j + 2);
+        if constexpr (NS == 3) {
+            if (j + 1 < steps) make_tiles(mb, j + 1);
+        }
         // PRE = false always branches here (in one piece with the digits below, the compiler spills registers)
         if ((KS == 1 && PRE) || j < cnt_) products(sb, sc);
-        if constexpr (!PRE) {
-            stage_tiles(v, nb, s ^ 1);
+        if constexpr (NS == 2) {
+            if (j + 1 < steps) make_tiles(nb, j + 1);
         }
         if (wide) {
             // rare: the remainders of the blocks that need them take the tiles' place
             __syncthreads();
-            load_x(g, v);
-            make_second(v, sb);
+            make_second(g, sb);
             __syncthreads();
             if (KS == 1 || j < cnt) products(sb, sc);
         }
     };
-    for (int j = 0; j < steps; j += 2) {
-        step(j, st0, st1, 0);
-        if (j + 1 < steps) step(j + 1, st1, st0, 1);
+    if constexpr (PRE) {
+        uint8_t* const st0 = lds0 + ks * STAGE;
+        uint8_t* const st1 = lds1 + ks * STAGE;
+        issue(group(0), st0, 0);
+        for (int j = 0; j < steps; j += 2) {
+            step(j, st0, nullptr, st1);
+            if (j + 1 < steps) step(j + 1, st1, nullptr, st0);
+        }
+    } else {
+        uint8_t* s0 = lds0 + ks * STAGE;
+        uint8_t* s1 = s0 + KS * STAGE;
+        uint8_t* s2 = NS == 3 ? s1 + KS * STAGE : s0;
+        issue(group(0), s0, 0);
+        if (NS == 3) issue(group(1), s1, 1);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        make_tiles(s0, 0);
+#pragma unroll 1
+        for (int j = 0; j < steps; ++j) {
+            step(j, s0, s1, NS == 3 ? s2 : s1);
+            uint8_t* const t = s0;
+            s0 = s1;
+            s1 = NS == 3 ? s2 : t;
+            s2 = t;
+        }
     }
     // the last copies (repeats into free stages) land before the block's LDS is reused or released
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -113,3 +113,38 @@ def test_small_columns_beside_large_ones(gpu, large, mag):
             got = call(torch, ctx, [(w, s, codes)], x, work)[0]
             worst = float(np.max(np.abs(got - ref) / tol))
             assert worst <= 1, f"workspace {work}: {worst:.2f} of the bound"
+
+
+# without a workspace: 32 x 512 blocks (an odd number of groups, rows of three matrices), 64 x 512 blocks, full rounds of
+# those and 32 x 512 blocks for the last 100 tokens, and for the last one
+@pytest.mark.parametrize("T,K", [(700, 384), (1025, 128), (1700, 256), (1601, 128)])
+def test_in_place_blocks(gpu, T, K):
+    """Calls that add into strided outputs, with LoRA rows and a strided x: the same bits with and without a workspace,
+    and within workload.ternary_tolerance of float64 (and of 1e-6 of the LoRA part, 16 fp32 products)."""
+    torch, ctx, _ = gpu
+    os, r, pad = (4096, 512, 512), 16, 8
+    print(f"ternary in place T={T} K={K}", flush=True)
+    mats = [workload.ternary_weights(0x7D00 + i, o, K, True) for i, o in enumerate(os)]
+    x = oracle.normal(0x7D00 + T, 1, (T, K + pad)).copy()
+    y0 = [oracle.normal(0x7D10 + i, 2, (T, o + 4)) for i, o in enumerate(os)]
+    lu = oracle.normal(0x7D20, 3, (T, 3 * r + 5))
+    lb = [oracle.f32_to_f16(oracle.normal(0x7D30 + i, 4, (o, r))) for i, o in enumerate(os)]
+    xd, lud = dev(torch, x)[:, :K], dev(torch, lu)
+    packed = [(dev(torch, w.view(np.int32)), dev(torch, s.view(np.int16))) for w, s, _ in mats]
+    lbd = [dev(torch, b.view(np.int16)) for b in lb]
+    got = []
+    for work in (True, False):
+        ys = [dev(torch, y) for y in y0]
+        ba.ternary_matmul(ctx, xd, [(w, s, y[:, :o], b) for (w, s), y, o, b in zip(packed, ys, os, lbd)], add=True,
+                          lora_u=lud, lora_r=r, work=ba.ternary_workspace(xd) if work else None)
+        torch.cuda.synchronize()
+        got.append([y.cpu().numpy() for y in ys])
+    for i, ((w, s, codes), o) in enumerate(zip(mats, os)):
+        a, b = got[0][i], got[1][i]
+        assert np.array_equal(a, b), f"matrix {i}"
+        assert np.array_equal(a[:, o:], y0[i][:, o:]), "columns beside the matrix"
+        full = (codes.astype(np.float64) - 1) * np.repeat(oracle.f16_to_f32(s).astype(np.float64), 128, axis=1)
+        u, B = lu[:, i * r:(i + 1) * r].astype(np.float64), oracle.f16_to_f32(lb[i]).astype(np.float64)
+        ref = x[:, :K].astype(np.float64) @ full.T + u @ B.T + y0[i][:, :o]
+        tol = workload.ternary_tolerance(x[:, :K], codes, s) + 1e-6 * (np.abs(u) @ np.abs(B).T + np.abs(y0[i][:, :o]))
+        assert (np.abs(a[:, :o] - ref) <= tol).all(), f"matrix {i}"
