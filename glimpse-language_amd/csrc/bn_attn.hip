@@ -612,7 +612,7 @@ bn_status run_prefill(bn_ctx* ctx, hipStream_t st, const bn_attn_args* a, const 
             bn_launch(ctx, (bn::prefill_hilo_kernel<true, true>), dim3((unsigned)blocks), dim3(256), 0, st, f);
         bn_status s = launched(ctx, "prefill_hilo_kernel (split)");
         if (s) return s;
-        bn_launch(ctx, bn::prefill_combine_kernel, dim3(a->T, 2 * a->KV), dim3(64), 0, st, f);
+        bn_launch(ctx, bn::prefill_combine_kernel, dim3(a->T, 2 * a->KV), dim3(128), 0, st, f);
         return launched(ctx, "prefill_combine_kernel");
     }
     if (split) {

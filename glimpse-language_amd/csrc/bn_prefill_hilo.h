@@ -427,108 +427,108 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 }
 
 // Merge of the key splits of one (token, head pair) in split order (attn_combine.comp:10-20), then the gate and, with
-// signs, the rotation of the pair's 512 elements (gate_rotate.comp:18-25). Grid (T, H / 2) x 64 threads; thread: dims
-// 4 lane .. +3 of both heads. Bound by the records' round trips: the first 8 splits' accumulators are requested with
-// the (m, l) terms.
-__global__ __launch_bounds__(64) void prefill_combine_kernel(PrefillArgs a) {
-    constexpr int PRE = 8;
-    const int t = blockIdx.x, lane = threadIdx.x, kh = blockIdx.y >> 1, p = blockIdx.y & 1;
+// signs, the rotation of the pair's 512 elements (gate_rotate.comp:18-25). Grid (T, H / 2) x 128 threads; a wave per head,
+// thread: dims 4 lane .. +3 of it; with signs the second head's row goes through LDS to the first's wave, which transforms
+// the pair. Bound by the records' round trips: the first 16 splits' accumulators are requested with the (m, l) terms, the
+// others 8 at a time (one wave for both heads, the first 8 up front and the others one by one, took 12 us instead of 6 for
+// 96 rows over 1,031, 18 splits, 8/2 heads).
+__global__ __launch_bounds__(128) void prefill_combine_kernel(PrefillArgs a) {
+    constexpr int PRE = 16, FEW = 8;
+    __shared__ f4 row1[64];
+    const int t = blockIdx.x, lane = threadIdx.x & 63, kh = blockIdx.y >> 1, p = blockIdx.y & 1;
+    const int i = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);  // head of the pair
     const int qt = t / PF_BQ, t_last = min(a.T, qt * PF_BQ + PF_BQ) - 1;
     const int hd = kh * 4 + 2 * p;  // the pair's first head
-    f4 z[2], sg[2];
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        z[i] = sg[i] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (a.gate)
-            z[i] = *reinterpret_cast<const f4*>(a.gate + (int64_t)t * a.g_ts + (int64_t)(hd + i) * a.g_hs + 4 * lane);
-        if (a.signs) sg[i] = *reinterpret_cast<const f4*>(a.signs + (int64_t)(hd + i) * D + 4 * lane);
-    }
+    f4 z = {0.0f, 0.0f, 0.0f, 0.0f}, sg = z;
+    if (a.gate) z = *reinterpret_cast<const f4*>(a.gate + (int64_t)t * a.g_ts + (int64_t)(hd + i) * a.g_hs + 4 * lane);
+    if (a.signs) sg = *reinterpret_cast<const f4*>(a.signs + (int64_t)(hd + i) * D + 4 * lane);
     const int ns = pf_splits((call_off(a.dyn, a.off) + t_last + PF_BK) / PF_BK, a.ct);
-    // row of split 0, head 2 p; head i is PF_BQ rows on, split s PF_ROWS rows
-    const int64_t row0 = ((int64_t)kh * a.ntq + qt) * a.max_splits * PF_ROWS + 2 * p * PF_BQ + t % PF_BQ;
-    auto acc_of = [&](int s, int i) {
-        return *reinterpret_cast<const f4*>(a.part_acc + (row0 + (int64_t)s * PF_ROWS + i * PF_BQ) * D + 4 * lane);
+    // row of the head's split 0; split s is PF_ROWS rows on
+    const int64_t row0 = ((int64_t)kh * a.ntq + qt) * a.max_splits * PF_ROWS + (2 * p + i) * PF_BQ + t % PF_BQ;
+    auto acc_of = [&](int s) {
+        return *reinterpret_cast<const f4*>(a.part_acc + (row0 + (int64_t)s * PF_ROWS) * D + 4 * lane);
     };
-    f4 pre[PRE][2];
+    const float* ml = a.part_ml + row0 * 2;
+    f4 pre[PRE];
 #pragma unroll
-    for (int u = 0; u < PRE; u++)
+    for (int u = 0; u < PRE; u++) pre[u] = u < ns ? acc_of(u) : f4{0.0f, 0.0f, 0.0f, 0.0f};
+    float L = 0.0f;
+    f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (ns <= FEW) {
+        // few splits: every lane takes all their terms, without the exchanges below
+        float m[FEW], l[FEW];
 #pragma unroll
-        for (int i = 0; i < 2; i++) pre[u][i] = u < ns ? acc_of(u, i) : f4{0.0f, 0.0f, 0.0f, 0.0f};
-    float y[8];
+        for (int u = 0; u < FEW; u++) {
+            const float* r = ml + (int64_t)min(u, ns - 1) * PF_ROWS * 2;
+            m[u] = u < ns ? r[0] : -INFINITY;
+            l[u] = r[1];
+        }
+        float M = m[0];
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const float* ml = a.part_ml + (row0 + i * PF_BQ) * 2;
-        float L = 0.0f;
-        f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (ns <= PRE) {
-            // few splits: every lane takes all their terms, without the exchanges below
-            float m[PRE], l[PRE];
+        for (int u = 1; u < FEW; u++) M = fmaxf(M, m[u]);
 #pragma unroll
-            for (int u = 0; u < PRE; u++) {
-                const float* r = ml + (int64_t)min(u, ns - 1) * PF_ROWS * 2;
-                m[u] = u < ns ? r[0] : -INFINITY;
-                l[u] = r[1];
+        for (int u = 0; u < FEW; u++) {
+            const float wu = m[u] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[u] - M);
+            L = fmaf(l[u], wu, L);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[e] = fmaf(pre[u][e], wu, acc[e]);
+        }
+    } else {
+        auto m_of = [&](int s) { return s < ns ? ml[(int64_t)s * PF_ROWS * 2] : -INFINITY; };
+        auto l_of = [&](int s) { return s < ns ? ml[(int64_t)s * PF_ROWS * 2 + 1] : 0.0f; };
+        const float m0 = m_of(lane), l0 = l_of(lane);
+        float M = m0;
+        for (int s = lane + 64; s < ns; s += 64) M = fmaxf(M, m_of(s));
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
+        for (int base = 0; base < ns; base += 64) {
+            const float ms = base == 0 ? m0 : m_of(base + lane), ls = base == 0 ? l0 : l_of(base + lane);
+            const float wgt = ms == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms - M);  // split base + lane
+            const int cnt = min(64, ns - base);
+            auto add = [&](int u, f4 v) {
+                const float wu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), u));
+                L = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(ls), u)), wu, L);
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[e] = fmaf(v[e], wu, acc[e]);
+            };
+            int u0 = 0;
+            if (base == 0) {
+#pragma unroll
+                for (int u = 0; u < PRE; u++)
+                    if (u < cnt) add(u, pre[u]);
+                u0 = PRE;
             }
-            float M = m[0];
+            for (; u0 < cnt; u0 += 8) {
+                f4 v[8];
 #pragma unroll
-            for (int u = 1; u < PRE; u++) M = fmaxf(M, m[u]);
+                for (int u = 0; u < 8; u++)
+                    if (u0 + u < cnt) v[u] = acc_of(base + u0 + u);
 #pragma unroll
-            for (int u = 0; u < PRE; u++) {
-                const float wu = m[u] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[u] - M);
-                L = fmaf(l[u], wu, L);
-#pragma unroll
-                for (int e = 0; e < 4; e++) acc[e] = fmaf(pre[u][i][e], wu, acc[e]);
-            }
-        } else {
-            auto m_of = [&](int s) { return s < ns ? ml[(int64_t)s * PF_ROWS * 2] : -INFINITY; };
-            const float m0 = m_of(lane), l0 = lane < ns ? ml[(int64_t)lane * PF_ROWS * 2 + 1] : 0.0f;
-            float M = m0;
-            for (int s = lane + 64; s < ns; s += 64) M = fmaxf(M, m_of(s));
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
-            for (int base = 0; base < ns; base += 64) {
-                const int s_ = base + lane;
-                float ms = m0, ls = l0;
-                if (base > 0) {
-                    ms = m_of(s_);
-                    ls = s_ < ns ? ml[(int64_t)s_ * PF_ROWS * 2 + 1] : 0.0f;
-                }
-                const float wgt = ms == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms - M);  // split base + lane
-                const int cnt = min(64, ns - base);
-                auto add = [&](int u, f4 v) {
-                    const float wu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), u));
-                    L = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(ls), u)), wu, L);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) acc[e] = fmaf(v[e], wu, acc[e]);
-                };
-                int u0 = 0;
-                if (base == 0) {
-#pragma unroll
-                    for (int u = 0; u < PRE; u++)
-                        if (u < cnt) add(u, pre[u][i]);
-                    u0 = PRE;
-                }
-                for (; u0 < cnt; u0++) add(u0, acc_of(base + u0, i));
+                for (int u = 0; u < 8; u++)
+                    if (u0 + u < cnt) add(u0 + u, v[u]);
             }
         }
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            float v = acc[e] / L;
-            if (a.gate) v = gate_mul(v, z[i][e]);
-            y[4 * i + e] = v;
-        }
     }
-    float* o = a.out + (int64_t)t * a.o_ts + (int64_t)hd * a.o_hs + 4 * lane;
-    float scale = 1.0f;
-    if (a.signs) {
+    f4 y;
 #pragma unroll
-        for (int e = 0; e < 8; e++) y[e] *= sg[e >> 2][e & 3];
-        fwht512_wave(y, lane);
-        scale = INV_SQRT512;
+    for (int e = 0; e < 4; e++) {
+        y[e] = acc[e] / L;
+        if (a.gate) y[e] = gate_mul(y[e], z[e]);
     }
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-        *reinterpret_cast<f4*>(o + i * a.o_hs) = f4{y[4 * i], y[4 * i + 1], y[4 * i + 2], y[4 * i + 3]} * scale;
+    f4* const o = reinterpret_cast<f4*>(a.out + (int64_t)t * a.o_ts + (int64_t)(hd + i) * a.o_hs + 4 * lane);
+    if (!a.signs) {
+        *o = y;
+        return;
+    }
+    y *= sg;
+    if (i) row1[lane] = y;
+    __syncthreads();
+    if (i) return;
+    const f4 y1 = row1[lane];
+    float v[8] = {y[0], y[1], y[2], y[3], y1[0], y1[1], y1[2], y1[3]};
+    fwht512_wave(v, lane);
+    *o = f4{v[0], v[1], v[2], v[3]} * INV_SQRT512;
+    *reinterpret_cast<f4*>(reinterpret_cast<float*>(o) + a.o_hs) = f4{v[4], v[5], v[6], v[7]} * INV_SQRT512;
 }
 
 }  // namespace bn
