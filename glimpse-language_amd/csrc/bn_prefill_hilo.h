@@ -25,6 +25,8 @@
 // (MI355X, a layer call, fp32 q): 777 rows over 1,031, 16/4 heads 121 -> 71 us; 500 over 517, 8/2 53 -> 36; 1,900 over 4,000,
 // 16/4 492 -> 287; 3,000 over 1,000, 8/2 239 -> 161.
 #pragma once
+#include <type_traits>
+
 #include "bn_prefill.h"
 
 namespace bn {
@@ -218,12 +220,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         }
     }
 
-    // Tile j: S^T(j + 1) from stage j + 1 (computed also after the last tile, from a stage whose copies are done,
-    // and dropped), P(j) from S^T(j), O += P(j) V(j) from stage j.
-    for (int j = jb; j < nt; j++) {
+    // Tile j: S^T(j + 1) from stage j + 1 (MORE; the kernel without splits computes it also after the last tile, from a
+    // stage whose copies are done, and drops it), P(j) from S^T(j), O += P(j) V(j) from stage j.
+    auto tile_step = [&](int j, auto copy, auto more) __attribute__((always_inline)) {
+        constexpr bool COPY = decltype(copy)::value, MORE = decltype(more)::value;
         // tile j + 1 landed (tile j + 2's copies may be in flight), and every wave is done with tile j - 1, whose
         // stage takes tile j + 3 (a repeat of the last tile past the end), copied during the S^T(j + 1) MFMAs below
-        asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
+        if (COPY || j + 2 < nt)
+            asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
         const int jc = min(j + 3, nt - 1), js = j - jb;
         uint8_t* cst = lds + ((js + 3) & (PH_STAGES - 1)) * PF_STAGE;
         const uint8_t* cur = lds + (js & (PH_STAGES - 1)) * PF_STAGE;
@@ -234,7 +240,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         const uint8_t* kl = nxt + k_lane;
         h8 kop[16];
 #pragma unroll
-        for (int ks = 0; ks < KA; ks++) kop[ks] = pf_lds_h8(kl + ks * 32);
+        for (int ks = 0; ks < KA; ks++)
+            if (MORE) kop[ks] = pf_lds_h8(kl + ks * 32);
 
         // the row max of S(j); causal mask on tiles that cross the diagonal (register r: key j0 + 8 (r/4) + 4 h + r%4)
         const int j0 = j * PF_BK;
@@ -297,17 +304,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         // the reads stay KA (V: VA) steps ahead; left alone, the compiler moves each read next to its MFMA.
 #pragma unroll
         for (int ks = 0; ks < 16; ks++) {
-            if (ks + KA < 16) kop[ks + KA] = pf_lds_h8(kl + (ks + KA) * 32);
+            if (MORE && ks + KA < 16) kop[ks + KA] = pf_lds_h8(kl + (ks + KA) * 32);
             if (ks + VA >= 16) v_read(ks + VA - 16);
-            s_next = mfma32(kop[ks], qb[ks], s_next);
-            if constexpr (HILO) s_next = mfma32(kop[ks], ql[ks], s_next);
+            if constexpr (MORE) {
+                s_next = mfma32(kop[ks], qb[ks], s_next);
+                if constexpr (HILO) s_next = mfma32(kop[ks], ql[ks], s_next);
+            }
             pa[ks >> 3][ks & 7] = (_Float16)__builtin_amdgcn_exp2f(fmaf(s_cur[ks], sc, -m_use));
+            if constexpr (!MORE) continue;
             if (ks + KA < 16 && ks + VA >= 16) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
             else if (ks + KA < 16) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             else if (ks + VA >= 16) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
             __builtin_amdgcn_sched_group_barrier(0x008, HILO ? 2 : 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x402, 4, 0);
-            if (ks & 1) {  // one copy after every second k-step's MFMAs, which stay ahead of it
+            if (COPY && (ks & 1)) {  // one copy after every second k-step's MFMAs, which stay ahead of it
                 tile_copy(jc, cst, ks >> 1);
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -331,6 +341,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         }
         s_cur = s_next;
+    };
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    if constexpr (SPLIT) {
+        // ranges are short: their last three tiles bring no others, and the last computes no further S (300 rows over 100,
+        // 16/4 heads, fp16 q, with the records' stores below: kernel 18.2 -> 15.2 us)
+        int j = jb;
+        for (; j < nt - 3; j++) tile_step(j, yes, yes);
+        for (; j < nt - 1; j++) tile_step(j, no, yes);
+        tile_step(j, no, no);
+    } else {
+        for (int j = jb; j < nt; j++) tile_step(j, yes, yes);
     }
 
     // Epilogue. O / l goes to LDS as each wave's [32 tokens][256 dims] (pitch PH_OP), then rows are read back 16
@@ -378,10 +400,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             a.part_ml[(row + r32) * 2] = m_run;
             a.part_ml[(row + r32) * 2 + 1] = l_tot;
         }
+        // Short ranges end together, and their stores with them: non-temporal, these leave the L2s at once instead of at the
+        // kernel's end (96 rows over 512, 32/8 heads, 20 MB: kernel 20.2 -> 18.7 us, the merge 0.4 longer). Not where
+        // longer ranges end apart anyway, nor where the merge reads a row's splits in several round trips (65 rows over
+        // 5,000, one kv head: 36 us, 41 with them).
+        float* const rec = a.part_acc + row * D + 4 * lane;
+        const uint8_t* const src = orow + 16 * lane;
+        if (a.ct <= 8 && a.max_splits <= 16) {
 #pragma unroll 4
-        for (int tl = 0; tl < PF_BQ; tl++)
-            *reinterpret_cast<f4*>(a.part_acc + (row + tl) * D + 4 * lane) =
-                *reinterpret_cast<const f4*>(orow + tl * PH_OP + 16 * lane);
+            for (int tl = 0; tl < PF_BQ; tl++)
+                __builtin_nontemporal_store(*reinterpret_cast<const f4*>(src + tl * PH_OP), reinterpret_cast<f4*>(rec + tl * D));
+        } else {
+#pragma unroll 4
+            for (int tl = 0; tl < PF_BQ; tl++)
+                *reinterpret_cast<f4*>(rec + tl * D) = *reinterpret_cast<const f4*>(src + tl * PH_OP);
+        }
         return;
     }
     if (!a.signs) {
