@@ -245,6 +245,8 @@ bn_status check_lora(const uint16_t* A, const float* U, int64_t u_ts, uint32_t r
     return BN_OK;
 }
 
+size_t workspace_need(const bn_attn_args* a);
+
 bn_status check_attn(const bn_attn_args* a, int kind, char* why) {
     if (!a) return set_err(why, BN_EINVAL, "args is NULL");
     if (kind < 0 || kind > 4) return set_err(why, BN_EINVAL, "unknown kind %d", kind);
@@ -280,7 +282,7 @@ bn_status check_attn(const bn_attn_args* a, int kind, char* why) {
     if (a->signs && !aligned16(a->signs)) return set_err(why, BN_EINVAL, "signs must be 16-byte aligned");
     bn_status ls = check_lora(a->lora_a, a->lora_u, a->lora_us, a->lora_r, a->T, (int64_t)a->H * bn::D, bn::LORA_MAX_K, why);
     if (ls) return ls;
-    size_t need = bn_attn_workspace_size(a);
+    const size_t need = workspace_need(a);
     if (need && (!a->ws || a->ws_bytes < need || !aligned16(a->ws)))
         return set_err(why, BN_ENOWS, "workspace needs %zu bytes (16-byte aligned), got %zu", need, a->ws_bytes);
     return BN_OK;
@@ -657,6 +659,55 @@ int64_t mid_chunk(const bn_attn_args* a) {
 size_t mid_records_bytes(const bn_attn_args* a) {
     const int64_t T = a->T, ns = ceil_div((int64_t)a->off + T, mid_chunk(a));
     return (size_t)(a->KV * 8 * T * ceil_div(ns, 8)) * bn::DEC_PART * sizeof(float);
+}
+
+// The workspace bytes that a call needs. The kernel choice for T >= 2 depends on the context, so this covers the split key
+// ranges' records and, for more than 16 rows, verify_kernel's row-group records.
+size_t workspace_need(const bn_attn_args* a) {
+    size_t rows = a->T <= (uint32_t)kVerifyMax ? plan_rows(a, 1, BN_DECODE_MAX_TARGET_WAVES, kMaxSplitsCap).total() : 0;
+    if (verify_chunk(a)) rows = verify_q_offset(a) + (size_t)a->T * a->H * bn::D * sizeof(float);
+    if (a->T == 1) return rows;
+    size_t fl = plan_split(a->T, a->off, a->KV).total();
+    if (a->T > (uint32_t)kVerifyMax && a->T <= kMidMaxRows) {
+        const size_t mid = mid_records_bytes(a);
+        if (mid > fl) fl = mid;
+    }
+    return fl > rows ? fl : rows;
+}
+
+// The most that workspace_need gives for 1..T rows over 0..off cached rows. A plan's records don't grow with the sizes (a
+// fresh prompt's uneven q-tiles take more splits than the same rows over a long prefix, a chunk that fills the GPU takes
+// none), so a workspace for a conversation is sized by bounds:
+//  - up to 16 rows: the plan for a device offset, which covers every smaller one, and the fp32 q rows after it;
+//  - 17..64: the splits that kMidTargetBlocks allows, of 128 keys at least;
+//  - q-tiles: with M splits of the longest, the N q-tiles of all kv heads have N M / 2 or more in all (their lengths grow by
+//    a tile each), and no more than kSplitTarget if any is split, so M <= 2 kSplitTarget / N; of 2 key tiles at least.
+size_t workspace_bound(const bn_attn_args* a) {
+    static const uint32_t any_offset = 0;
+    const int64_t KV = a->KV, off = a->off;
+    size_t most = 0;
+    auto take = [&](size_t n) { most = n > most ? n : most; };
+    bn_attn_args p = *a;
+    p.dyn = &any_offset;
+    for (uint32_t t = 1; t <= a->T && t <= (uint32_t)kVerifyMax; t++) {
+        p.T = t;
+        const DecodePlan d = plan_rows(&p, 1, BN_DECODE_MAX_TARGET_WAVES, kMaxSplitsCap);
+        size_t n = d.total();
+        if (t == 1 && !a->dyn) n = d.units > 1 ? n / d.slots * d.units : 0;  // one slot per unit
+        take(n && t > 1 ? (n + 255) / 256 * 256 + (size_t)t * a->H * bn::D * sizeof(float) : n);
+    }
+    for (int64_t t = kVerifyMax + 1; t <= (int64_t)a->T && t <= (int64_t)kMidMaxRows; t++) {
+        const int64_t by_blocks = ceil_div(kMidTargetBlocks, KV * ceil_div(t, 8));
+        const int64_t by_keys = ceil_div(off + t, 32 * BN_VERIFY_WAVES);
+        take((size_t)(KV * 8 * t * ceil_div(by_blocks < by_keys ? by_blocks : by_keys, 8)) * bn::DEC_PART * sizeof(float));
+    }
+    for (int64_t q = 1, n = KV; a->T > 1 && n < kSplitTarget && q <= ceil_div(a->T, bn::PF_BQ); q++, n += KV) {
+        const int64_t rows = q * bn::PF_BQ < (int64_t)a->T ? q * bn::PF_BQ : a->T;
+        const int64_t by_blocks = 2 * kSplitTarget / n, by_keys = ceil_div(ceil_div(off + rows, bn::PF_BK), 2);
+        const int64_t m = by_blocks < by_keys ? by_blocks : by_keys;
+        if (m > 1) take((size_t)(n * m * bn::PF_ROWS) * (bn::D + 2) * sizeof(float));
+    }
+    return most;
 }
 
 bn_status run_tiles(bn_ctx* ctx, hipStream_t st, const bn_attn_args* a) {
@@ -1115,18 +1166,7 @@ void bn_ctx_destroy(bn_ctx* ctx) { delete ctx; }
 const char* bn_ctx_last_error(const bn_ctx* ctx) { return ctx ? ctx->err : g_check_err; }
 
 size_t bn_attn_workspace_size(const bn_attn_args* a) {
-    if (!a || a->KV < 1 || a->T < 1) return 0;
-    size_t rows = a->T <= (uint32_t)kVerifyMax ? plan_rows(a, 1, BN_DECODE_MAX_TARGET_WAVES, kMaxSplitsCap).total() : 0;
-    if (verify_chunk(a)) rows = verify_q_offset(a) + (size_t)a->T * a->H * bn::D * sizeof(float);
-    if (a->T == 1) return rows;
-    // the kernel choice for T >= 2 depends on the context, so the size covers the split key ranges' records and, for
-    // more than 16 rows, verify_kernel's row-group records
-    size_t fl = plan_split(a->T, a->off, a->KV).total();
-    if (a->T > (uint32_t)kVerifyMax && a->T <= kMidMaxRows) {
-        const size_t mid = mid_records_bytes(a);
-        if (mid > fl) fl = mid;
-    }
-    return fl > rows ? fl : rows;
+    return !a || a->KV < 1 || a->T < 1 ? 0 : workspace_bound(a);
 }
 
 size_t bn_ragged_workspace_size(const bn_ragged_args* a) {

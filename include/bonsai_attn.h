@@ -89,8 +89,7 @@ typedef struct bn_attn_args {
     const float* signs; /* [H * 256] +1/-1 (16-byte aligned), or NULL. When set, `out` receives o_proj's input
                            instead of the gated output: the rest of gate_rotate (gate_rotate.comp:22-25), i.e.
                            per row and block of 512 elements (heads 2j, 2j+1), H_512 (gated * signs) / sqrt(512).
-                           The attention kernels rotate in their epilogue (the fallback prefill kernel for
-                           calls too small to fill the GPU rotates in place after it). */
+                           The attention kernels rotate in their epilogue, or in the merge of split key ranges. */
 
     const uint32_t* dyn; /* NULL, or device memory holding this call's cache offset (the reference's dynamic
                             parameter slot for replayed command buffers: attn_split.comp:12-14, attn_prep.comp:32-33,
@@ -276,6 +275,9 @@ int bn_abi_version(void);
 bn_status bn_dyn_overflow(bn_ctx* ctx, int* flag);
 
 /* ---- sizes and checks (pure host code, no device access) ----------------------------------------- */
+/* Workspace bytes for any call of 1..T rows over 0..off cached rows of these heads: never less for more rows or a larger
+ * offset, so one workspace of the size for the most rows at the full context serves them all. (A call itself is refused
+ * only if its own plan needs more than it is given, which may be less or nothing.) */
 size_t bn_attn_workspace_size(const bn_attn_args* a);
 size_t bn_ragged_workspace_size(const bn_ragged_args* a);
 /* kind: 0 forward (any T), 1 decode (T == 1), 2 verify (T <= 16), 3 prefill (any T), 4 append only */

@@ -131,6 +131,29 @@ def test_device_offset_workspace_stays_near_the_exact_one(lib, T, H, KV, bound):
 
 
 
+@pytest.mark.parametrize("H,KV", [(4, 1), (8, 2), (16, 4), (32, 8), (12, 3)])
+def test_workspace_covers_smaller_calls(lib, H, KV):
+    """A workspace sized for T rows at an offset serves fewer rows and smaller offsets: the size never falls with either,
+    and every such call passes the check with it. (500 rows of 16/4 heads take 6 splits over no prefix, 4 over 1,024.)"""
+    rows = [1, 2, 3, 8, 16, 17, 33, 64, 65, 96, 130, 256, 333, 500, 777, 1000, 1500, 1987, 2040, 2100, 4000]
+    offs = [0, 1, 40, 100, 333, 517, 1024, 2000, 4095, 8192, 16384, 40000, 65536, 65600, 131000]
+
+    def args(T, off, ws_bytes=0):
+        a = good_args(T=T, off=off, H=H, KV=KV)
+        a.ws, a.ws_bytes = 0x200000, ws_bytes
+        return a
+
+    size = {(T, off): ba.workspace_size(args(T, off)) for T in rows for off in offs}
+    for i, T in enumerate(rows):
+        for j, off in enumerate(offs):
+            for t, o in ((rows[max(i - 1, 0)], off), (T, offs[max(j - 1, 0)])):
+                assert size[t, o] <= size[T, off], f"{t} rows over {o} against {T} over {off}"
+    for T, off in ((500, 40000), (4000, 131000), (64, 8192), (16, 65600), (1, 131000)):
+        for t in sorted({t for r in rows for t in (r, r - 1, r - 7) if 1 <= t <= T}):
+            for o in list(range(0, min(off, 2200), 13)) + [x for x in offs if x <= off] + [off - 1, off // 3]:
+                assert ba.check(args(t, o, size[T, off])) == ba.BN_OK, f"{t} rows over {o}, sized for {T} over {off}"
+
+
 def test_ragged_check(lib):
     r = ba.RaggedArgs()
     r.nseq, r.H, r.KV, r.max_len = 4, 8, 2, 100
