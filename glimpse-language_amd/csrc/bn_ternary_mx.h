@@ -15,15 +15,14 @@
 // Digits end at the same place for all 32 values, so columns far below a block's largest keep fewer bits of their own,
 // which a row whose weights are 0 on the large columns shows. Such a block's remainder is written as five more digits and
 // multiplied by a second pass over the group (flagged per 32-token tile; blocks that need none are zero there). It is
-// made where the digits of these columns do not end:
-//   - at least 12 of the block's columns within S 2^-5, or 6 within S 2^-7.7; or
-//   - a column within S 2^-5 in every token of the tile (of 8 tokens or more), as columns of another scale are.
-// With small columns in the same places for a tile's tokens their error is then at most 1e-6 of their norm, and 2.3e-6
-// for single tokens with up to 25 large columns of 32 (worst of 1 to 31 large columns, 8 to 10^5 times the others, weights
-// 0 under them; the digits alone: 3e-3). The rules are no wider because a step with a second pass takes more than
-// twice as long, and the blocks of a call that runs in one round wait for it: they take 1e-7 of the blocks of normally
-// distributed values for such (with 2e-5 of them calls of 1,000 to 2,000 tokens took 10-20% longer). The block scale covers fp32's exponents; a block with an infinity or a NaN gets the scale NaN,
-// and the token's outputs are NaN.
+// made where the digits of at least 12 of the block's columns within S 2^-5, or of 6 within S 2^-7.7, do not end: with up
+// to 25 large columns of 32 the others' error is then at most 2.3e-6 of their norm (worst of factors 8 to 10^5 between
+// them, weights 0 under the large ones; the digits alone: 3e-3, which fewer small columns keep). The rules are no wider
+// because a step with a second pass takes more than twice as long, and the blocks of a call that runs in one round wait
+// for it: they take 1e-7 of the blocks of normally distributed values for such (with 2e-5 of them calls of 1,000 to 2,000
+// tokens took 10-20% longer; a column that is small in all tokens of a tile says nothing, as tokens may be alike). The
+// block scale covers fp32's exponents; a block with an infinity or a NaN gets the scale NaN, and the token's outputs are
+// NaN.
 // Measured (MI355X, the 4B q/k/v projections of 4,096 tokens): 303 us (digits 17, GEMM 285) against 368 for the fp16
 // hi/lo split, whose 1.16 PFLOP/s of products were the rate of a large library product here; error against 64-bit sums
 // 1.1e-7 of the output's norm against 4.6e-7. The matrix units are busy two thirds of the time at the 1.7 GHz that the
@@ -92,41 +91,28 @@ __device__ __forceinline__ uint32_t tern_at_least(u6v w) {
     return r[0] | (r[1] >> 1);
 }
 __host__ __device__ constexpr int tern_bit(int e) { return (6 * (e & 15) + 5) % 32 - (e >> 4); }
-// OR over the 32 lanes of a lane's half
-__device__ __forceinline__ uint32_t or_half(uint32_t x) {
-    x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xF, 0xF, false);  // row_ror: 8, 4, 2, 1
-    x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x124, 0xF, 0xF, false);
-    x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x122, 0xF, 0xF, false);
-    x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x121, 0xF, 0xF, false);
-    const auto p = __builtin_amdgcn_permlane16_swap(x, x, false, false);
-    return p[0] | p[1];
-}
 // The digits of 32 values x of a token: each digit's six words through put(d, words). Returns the block's scale byte.
-// CHECK = false: x becomes the remainders. CHECK = true also tells in wide whether the block needs a second set of
-// digits (zeros for tokens past T; many: whether the tile has 8 tokens or more, lane: token lane % 32 of it).
+// CHECK = false: x becomes the remainders. CHECK = true: only where some block of the wave may need a second set of
+// digits; tells in wide whether this one does.
 template <bool CHECK, typename Put>
-__device__ __forceinline__ int tern_digits(TernBlock& x, bool many, bool& wide, const Put& put) {
+__device__ __forceinline__ int tern_digits(TernBlock& x, bool& wide, const Put& put) {
     float mx = 0.0f;  // an infinity or a NaN stays
 #pragma unroll
     for (int i = 0; i < 16; ++i) asm("v_maximum3_f32 %0, |%1|, |%2|, %0" : "+v"(mx) : "v"(x.u[i]), "v"(x.v[i]));
     const int eb = (__float_as_int(mx) >> 23) & 255;
     const int e = max(eb - 1, 28);  // 28: the last digit's scale stays normal
     // columns above S 2^-5, above S 2^-7.7: by the first two digits
-    uint32_t over[2], tile_over;
+    uint32_t over[2];
     bool ask = false;
 #pragma unroll
     for (int d = 0; d < TMX_ND; ++d) {
         const float sc = tern_pow2(e - 5 * d);
         const u6v q = __builtin_bit_cast(u6v, __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(x.u, x.v, sc));
         put(d, q);
-        if (CHECK && d == 0) {
-            over[0] = tern_at_least<1>(q);
-            tile_over = many ? or_half(over[0]) : 0xFFFFFFFFu;
-        }
+        if (CHECK && d == 0) over[0] = tern_at_least<1>(q);
         if (CHECK && d == 1) {
             over[1] = over[0] | tern_at_least<3>(q);
-            ask = mx != 0.0f && (__builtin_popcount(over[0]) <= 32 - 12 || __builtin_popcount(over[1]) <= 32 - 6 ||
-                                 tile_over != 0xFFFFFFFFu);
+            ask = mx != 0.0f && (__builtin_popcount(over[0]) <= 32 - 12 || __builtin_popcount(over[1]) <= 32 - 6);
         }
         if (CHECK && d == TMX_ND - 1 && __ballot(ask) == 0) break;
         const f32v b = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(q, sc);
@@ -146,8 +132,7 @@ __device__ __forceinline__ int tern_digits(TernBlock& x, bool many, bool& wide, 
                 rest |= x.u[i] != 0.0f ? 1u << tern_bit(2 * i) : 0u;
                 rest |= x.v[i] != 0.0f ? 1u << tern_bit(2 * i + 1) : 0u;
             }
-            wide = ask && (__builtin_popcount(rest & ~over[0]) >= 12 || __builtin_popcount(rest & ~over[1]) >= 6 ||
-                           (rest & ~tile_over) != 0);
+            wide = __builtin_popcount(rest & ~over[0]) >= 12 || __builtin_popcount(rest & ~over[1]) >= 6;
         }
     }
     return eb == 255 ? 255 : e;
@@ -224,8 +209,7 @@ __global__ __launch_bounds__(256, 4) void tern_digits_kernel(const float* __rest
         for (int i = 0; i < 16; ++i) v.u[i] = v.v[i] = 0.0f;
     }
     bool wide;
-    const int e = tern_digits<true>(v, T - t0 - 32 * u >= 8, wide,
-                                    [&](int d, u6v q) { tern_mx_put(out, kh, d, lane, q); });
+    const int e = tern_digits<true>(v, wide, [&](int d, u6v q) { tern_mx_put(out, kh, d, lane, q); });
     out[TMX_DIG + 4 * lane + kh] = (uint8_t)e;
     out[TMX_DIG + 4 * lane + 2 + kh] = wide;
     __shared__ int wide_lds[4];
@@ -374,7 +358,7 @@ __global__ __launch_bounds__(64 * W * KS, 2) void tern_mx_kernel(TernArgs a, int
             for (int c = 0; c < 16; ++c) v.u[c] = v.v[c] = 0.0f;
         }
         bool wide;
-        const int e = tern_digits<true>(v, a.T - tx >= 8, wide, [&](int d, u6v q) {
+        const int e = tern_digits<true>(v, wide, [&](int d, u6v q) {
             *reinterpret_cast<u4*>(dst + d * TMX_RDIG + 16 * lane) = u4{q[0], q[1], q[2], q[3]};
             *reinterpret_cast<u2*>(dst + d * TMX_RDIG + 1024 + 8 * lane) = u2{q[4], q[5]};
         });
@@ -397,7 +381,7 @@ __global__ __launch_bounds__(64 * W * KS, 2) void tern_mx_kernel(TernArgs a, int
         int e = 0;
 #pragma unroll 1
         for (int pass = 0; pass < 2; ++pass) {
-            e = tern_digits<false>(v, false, none, [&](int d, u6v q) {
+            e = tern_digits<false>(v, none, [&](int d, u6v q) {
                 if constexpr (PRE) {
                     tern_mx_put(dst, kh, d, lane, q);
                 } else {

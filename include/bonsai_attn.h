@@ -366,8 +366,8 @@ bn_status bn_ternary_check(const bn_ternary_args* a);
  * x's split error (the reference computes in fp32), identical from call to call, for any finite x up to about 4e9 in
  * magnitude (x beyond fp16's range is scaled by a power of two inside the call). The split error is 2^-22 of each value
  * up to 32 tokens. Beyond, it is 2^-24 of the largest of 32 neighbouring columns of a token, and 2^-48 of it where 12 or
- * more of the 32 lie 2^6 below that one, 6 or more 2^9, or a column lies 2^6 below it in all of the 8 to 32 tokens of a
- * tile. y must not overlap x, W or another matrix's y. */
+ * more of the 32 lie 2^6 below that one or 6 or more 2^9 (up to five columns beside 27 or more that are far larger keep
+ * 2^-24 of those). y must not overlap x, W or another matrix's y. */
 bn_status bn_ternary_matmul(bn_ctx* ctx, bn_stream stream, const bn_ternary_args* a);
 /* Bytes of bn_ternary_args.work for T tokens of width k (0 when T <= 32: those calls use none). With a workspace the
  * call runs two kernels: x split into its digits once, then the GEMM streaming those tiles; without, every block of the

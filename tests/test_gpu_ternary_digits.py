@@ -86,15 +86,14 @@ def test_digits_nonfinite_token(gpu):
         assert np.array_equal(got[rest], clean[rest])
 
 
-@pytest.mark.parametrize("large,mag", [(5, 1e3), (6, 1e4), (8, 30.0), (8, 2e4), (16, 300.0), (24, 1e3), (24, 1e5),
-                                       (28, 1e4), (31, 300.0), (31, 1e5)])
+@pytest.mark.parametrize("large,mag", [(5, 1e3), (6, 1e4), (8, 30.0), (8, 2e4), (16, 300.0), (20, 60.0), (24, 100.0),
+                                       (24, 1e3), (24, 1e5)])
 def test_small_columns_beside_large_ones(gpu, large, mag):
     """Some columns of every 32 (the same for all tokens, as channels of another scale are) hold values mag times the
     others', under weights 0: what is left are the small columns' products, to workload.ternary_tolerance (2e-5 of their
-    norm) as for any other call. Then with the large values in one token of 16 only, 24 of 32 columns at most (its own
-    columns decide there). T = 72: the last tile has 8 tokens."""
+    norm) as for any other call. Then with the large values in one token of 16 only."""
     torch, ctx, _ = gpu
-    T, K, O = 72, 768, 256
+    T, K, O = 70, 768, 256
     w, s, codes = workload.ternary_weights(0x7C00 + large, O, K, True)
     rank = np.argsort(np.argsort(oracle.normal(0x7C00 + large, 2, (K // 32, 32)), axis=1), axis=1).reshape(-1)
     big = rank < large
@@ -102,8 +101,6 @@ def test_small_columns_beside_large_ones(gpu, large, mag):
     w = workload.pack_codes(codes)
     base = oracle.normal(0x7C00 + large, 1, (T, K)).copy()
     for tokens in (np.arange(T), np.arange(3, T, 16)):
-        if len(tokens) < T and large > 24:
-            continue
         print(f"ternary digits, {large} of 32 columns x {mag} in {len(tokens)} tokens", flush=True)
         x = base.copy()
         x[np.ix_(tokens, big)] *= np.float32(mag)
