@@ -22,6 +22,16 @@
 #include "bn_util_kernels.h"
 #include "bn_verify.h"
 
+// The kernels of a decode step lie next to one another in the code object: with the prefill kernels' code between them a
+// whole layer's step of five launches (8K cached rows, 16/4 heads) took 36.6 us instead of 35.3, the same instructions.
+namespace bn {
+template __global__ void decode_split_kernel<1, false>(DecodeArgs);
+template __global__ void decode_split_kernel<2, true>(DecodeArgs);
+template __global__ void decode_split_kernel<2, false>(DecodeArgs);
+template __global__ void tern_rows_kernel<1, 1>(TernArgs);
+template __global__ void tern_rows_kernel<1, 2>(TernArgs);
+}  // namespace bn
+
 struct bn_ctx {
     int device;
     int cus;
