@@ -45,7 +45,7 @@ struct bn_ctx {
     int decode_target_waves;
     // splits of one sequence at most (1 .. kMaxSplitsCap; BONSAI_ATTN_DECODE_MAX_SPLITS)
     int decode_max_splits;
-    // blocks that split key ranges may give (1 .. kSplitTarget; BONSAI_ATTN_FLASH_TARGET_BLOCKS)
+    // blocks that split key ranges may give (1 .. kSplitTarget; BONSAI_ATTN_FLASH_TARGET_BLOCKS, any more as the most)
     int split_target_blocks;
     // 2..16 verify rows on verify_kernel (1, the default) or as decodes of their rows (0; BONSAI_ATTN_VERIFY_MFMA)
     int verify_mfma;
@@ -189,9 +189,10 @@ DecodePlan plan_rows(const bn_attn_args* a, int64_t waves, int64_t target_waves,
 // ceil(nt / ct) equal splits, ct the least number that gives no more blocks than that: a block costs a start (q rows,
 // the first tiles) and a 128 KB record besides about 2 us per key tile, so a second round of blocks loses more than it
 // balances (a layer call of 777 rows over 1,031, 16/4 heads: 67 us in one round, 85 with uneven shares for the XCDs).
-// At least 3 tiles a split, or 2 where that gives no more than half the blocks (256 rows over 512, 8/2 heads: 25.1
-// with 3, 26.0 with 4, 27.9 with 6; a layer call of 70 rows over none: 23.7 with 2, 28.2 unsplit). Depends only on the
-// shapes.
+// At least 3 tiles a split, or 2 where that gives no more than half the blocks (256 rows over 512, 8/2 heads: 26.9 us
+// with 3, 29.4 with 2, 26.4 with 4, 27.0 with 6; 400 over none, 16/4: 27.0 with 3 and 4, 27.8 with 2, 28.6 with 6; 65 over
+// 1,031, 4/1: 18.3 with 2 and 3, 19.4 with 4; a layer call of 70 rows over none: 22.1 with 2, 27.4 unsplit). Depends only
+// on the shapes.
 constexpr int64_t kSplitTarget = 256;
 
 struct SplitPlan {
@@ -1156,7 +1157,7 @@ bn_status bn_ctx_create(int device, bn_ctx** out) {
     c->split_target_blocks = (int)kSplitTarget;
     if (const char* e = getenv("BONSAI_ATTN_FLASH_TARGET_BLOCKS")) {
         const int v = atoi(e);
-        if (v >= 1 && v <= kSplitTarget) c->split_target_blocks = v;
+        if (v >= 1) c->split_target_blocks = v < kSplitTarget ? v : (int)kSplitTarget;
     }
     c->verify_mfma = 1;
     if (const char* e = getenv("BONSAI_ATTN_VERIFY_MFMA")) c->verify_mfma = atoi(e) != 0;

@@ -22,8 +22,9 @@
 // HILO = false is the same kernel on fp16 q, and SPLIT = true takes part of a q-tile's keys per block, for calls whose
 // q-tiles alone would leave CUs idle; prefill_combine_kernel merges the splits, gates and rotates. Against the kernel
 // with 64-key tiles, no pipelining and two separate launches for the merge and the rotation that these calls had
-// (MI355X, a layer call, fp32 q): 777 rows over 1,031, 16/4 heads 121 -> 71 us; 500 over 517, 8/2 53 -> 36; 1,900 over 4,000,
-// 16/4 492 -> 287; 3,000 over 1,000, 8/2 239 -> 161.
+// (MI355X, a layer call, fp32 q): 777 rows over 1,031, 16/4 heads 121 -> 70 us; 500 over 517, 8/2 53 -> 35; 1,900 over
+// 4,000, 16/4 492 -> 287; 3,000 over 1,000, 8/2 239 -> 161. Its sums differ from that kernel's within fp16 P's rounding: m per 32
+// keys, l over the rounded weights.
 #pragma once
 #include <type_traits>
 
@@ -322,6 +323,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        // l sums the weights as they multiply V, rounded, in fp32: rounding then moves sum and numerator alike (against 64
+        // bits, V of mean 1: 0.8-3.2e-5 of the output, with unrounded weights 1.1-4.6e-5; of mean 0 1.5-1.8e-4 both)
         const h2 one = {(_Float16)1.0f, (_Float16)1.0f};
 #pragma unroll
         for (int k = 0; k < 2; k++)
@@ -409,7 +412,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         if (a.ct <= 8 && a.max_splits <= 16) {
 #pragma unroll 4
             for (int tl = 0; tl < PF_BQ; tl++)
-                __builtin_nontemporal_store(*reinterpret_cast<const f4*>(src + tl * PH_OP), reinterpret_cast<f4*>(rec + tl * D));
+                __builtin_nontemporal_store(*reinterpret_cast<const f4*>(src + tl * PH_OP),
+                                            reinterpret_cast<f4*>(rec + tl * D));
         } else {
 #pragma unroll 4
             for (int tl = 0; tl < PF_BQ; tl++)
@@ -463,7 +467,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // signs, the rotation of the pair's 512 elements (gate_rotate.comp:18-25). Grid (T, H / 2) x 128 threads; a wave per head,
 // thread: dims 4 lane .. +3 of it; with signs the second head's row goes through LDS to the first's wave, which transforms
 // the pair. Bound by the records' round trips: the first 16 splits' accumulators are requested with the (m, l) terms, the
-// others 8 at a time (one wave for both heads, the first 8 up front and the others one by one, took 12 us instead of 6 for
+// others 8 at a time (one wave for both heads, the first 8 up front and the others one by one, took 11 us instead of 6 for
 // 96 rows over 1,031, 18 splits, 8/2 heads).
 __global__ __launch_bounds__(128) void prefill_combine_kernel(PrefillArgs a) {
     constexpr int PRE = 16, FEW = 8;

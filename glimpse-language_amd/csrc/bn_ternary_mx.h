@@ -25,7 +25,7 @@
 // NaN.
 // Measured (MI355X, the 4B q/k/v projections of 4,096 tokens): 303 us (digits 17, GEMM 285) against 368 for the fp16
 // hi/lo split, whose 1.16 PFLOP/s of products were the rate of a large library product here; error against 64-bit sums
-// 1.1e-7 of the output's norm against 4.6e-7. The matrix units are busy two thirds of the time at the 1.7 GHz that the
+// 0.9e-7 of the output's norm against 4.6e-7. The matrix units are busy two thirds of the time at the 1.7 GHz that the
 // power limit leaves (a loop of these MFMAs alone: 1.63 GHz, 157 us for this call's); without the copies the call took
 // 254 us, without the output stores 20 less, and neither another order of the loop nor more stages changed it.
 //
@@ -338,7 +338,8 @@ __global__ __launch_bounds__(64 * W * KS, 2) void tern_mx_kernel(TernArgs a, int
             } else {
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
-                    pf_copy16(xp[i & 3] + gb + (tx + 4 * i + (lane >> 4) < a.T ? i * row4 : 0), sb + mk * TMX_RAW + i * 1024);
+                    pf_copy16(xp[i & 3] + gb + (tx + 4 * i + (lane >> 4) < a.T ? i * row4 : 0),
+                              sb + mk * TMX_RAW + i * 1024);
             }
         }
     };
@@ -459,7 +460,8 @@ __global__ __launch_bounds__(64 * W * KS, 2) void tern_mx_kernel(TernArgs a, int
     for (int nt = 0; nt < 2; ++nt)                                                                              \
         t[nt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x0, b[nt][0], t[nt], 2, 4, 0, ex, DD, SW);      \
     for (int nt = 0; nt < 2; ++nt)                                                                              \
-        t[nt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x1, b[nt][1], t[nt], 2, 4, PRE ? 1 : 0, PRE ? ex : ex1, DD, SW)
+        t[nt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x1, b[nt][1], t[nt], 2, 4, PRE ? 1 : 0,         \
+                                                                PRE ? ex : ex1, DD, SW)
                 if (d == 4) { TMX_MFMA(0, sw1); }
                 if (d == 3) { TMX_MFMA(3, sw0); }
                 if (d == 2) { TMX_MFMA(2, sw0); }

@@ -166,8 +166,9 @@ def test_verify_kernel_equals_rows_path(gpu, T):
 @pytest.mark.parametrize("T,off,H,KV", [(40, 3000, 16, 4), (64, 100, 8, 2), (17, 0, 4, 1)])
 def test_mid_rows_equal_flash(gpu, T, off, H, KV):
     """17..64 rows take verify_kernel's row groups of 8 (BONSAI_ATTN_MID_ROWS, on by default) instead of
-    flash_kernel: both against the oracle, and against each other within 2e-4 (both carry an fp32 q as an fp16 hi/lo
-    pair; they differ in the order of the sums)."""
+    q-tiles on prefill_hilo_kernel (the key range split where that gives more blocks): both against the oracle, and
+    against each other within 2e-4 (both carry an fp32 q as an fp16 hi/lo pair; they differ in the order of the
+    sums)."""
     from conftest import context_with
     torch, ctx, ws = gpu
     inp = workload.layer(0x9700 + T + off, T=T, off=off, H=H, KV=KV)

@@ -148,9 +148,9 @@ def test_verify_peaky_scores(gpu, w, T, off, H, KV):
 @pytest.mark.parametrize("T,off,H,KV", [(256, 512, 8, 2), (512, 0, 16, 4)])
 def test_prefill_peaky_scores(gpu, w, T, off, H, KV, q16, path):
     """Prefill rows at peaky scores: within 2e-3 of the oracle, argmax equal. With q16 the query rows are given as
-    fp16 (BN_Q_F16, the oracle sees the same fp16 values); otherwise as fp32, which flash_kernel<true> and
-    prefill_hilo_kernel multiply as fp16 hi + lo parts. path "prefill" lowers the block threshold so these shapes run
-    on the prefill kernels (prefill_kernel for fp16 q, prefill_hilo_kernel for fp32 q) instead of flash_kernel."""
+    fp16 (BN_Q_F16, the oracle sees the same fp16 values); otherwise as fp32, which prefill_hilo_kernel multiplies as
+    fp16 hi + lo parts. path "flash": split key ranges on prefill_hilo_kernel, as calls this small run by default;
+    "prefill" lowers the block threshold so that they run whole, on prefill_kernel (fp16 q) or prefill_hilo_kernel."""
     torch = gpu[0]
     if path == "prefill":
         ctx = context_with(BONSAI_ATTN_PREFILL_MIN_BLOCKS=1)

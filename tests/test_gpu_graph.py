@@ -100,8 +100,8 @@ def test_decode_layer_graph_replay(gpu):
 
 
 # (T, off, off_max, H, KV, kind, min prefill blocks, fp16 q): decode (one split and many), verify rows on the MFMA
-# kernel, 12 rows as decodes of their rows, prefill on flash_kernel, prefill_hilo_kernel (fp32 q) and prefill_kernel
-# (fp16 q)
+# kernel, 12 rows as decodes of their rows, prefill on q-tiles with split keys, prefill_hilo_kernel (fp32 q) and
+# prefill_kernel (fp16 q)
 @pytest.mark.parametrize("T,off,off_max,H,KV,kind,min_blocks,q16", [
     (1, 40, 5000, 8, 2, ba.KIND_DECODE, 0, False),
     (1, 3000, 9000, 16, 4, ba.KIND_DECODE, 0, False),
@@ -196,7 +196,7 @@ def test_layer_device_offset_past_the_bound_appends_nothing(gpu):
 # (T, off, off_max, H, KV, rotate, min prefill blocks): the one-call layer (bn_attn_layer) with a device offset below
 # the host bound on its paths past one row: 8 verify rows (prep_kernel<8, 3> writes q and the K/V rows, then
 # verify_kernel and the merge), 12 rows (prep_kernel, then decodes of their rows with q normed in the prologue), a
-# prefill on flash_kernel and one on prefill_hilo_kernel (prep_kernel<4, 4> writes the fp32 q scratch)
+# prefill on q-tiles with split keys and one on whole q-tiles (prep_kernel<4, 4> writes the fp32 q scratch)
 @pytest.mark.parametrize("T,off,off_max,H,KV,rotate,min_blocks", [
     (8, 2048, 4000, 8, 2, True, 0),
     (12, 700, 2000, 8, 2, False, 0),

@@ -6,7 +6,7 @@ the same code, but inlined into another kernel the compiler may contract a produ
 the oracle's chain (oracle prep, oracle attention, oracle gate_rotate): max-abs 2e-3 and the same projected
 argmax. Cases cover every path of the call: one decode row (prep fused into the split kernel, which also appends
 the new K/V row), verify rows (K/V rows by prep_kernel, q in the split kernel's prologue), and prefills through
-prefill_kernel and through flash_kernel (q written by prep_kernel to the caller's scratch, fp32 or fp16).
+prefill_kernel and through q-tiles with split keys (q written by prep_kernel to the caller's scratch, fp32 or fp16).
 """
 import numpy as np
 import pytest
@@ -88,7 +88,7 @@ def check_layer(g, T, off, H, KV, rotate, seed, q16=False):
     (1, 9000, 16, 4, True),     # late position, many splits, rotated in the merge
     (8, 1000, 8, 2, True),      # verify rows
     (16, 3, 8, 2, False),
-    (200, 300, 8, 2, True),     # small prefill: flash_kernel reads the q that prep_kernel wrote
+    (200, 300, 8, 2, True),     # small prefill: q-tiles with split keys read the q that prep_kernel wrote
 ])
 def test_layer_matches_separate_calls_and_oracle(gpu, T, off, H, KV, rotate):
     check_layer(gpu, T, off, H, KV, rotate, 0xD000 + T + off)

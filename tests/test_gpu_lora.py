@@ -108,7 +108,7 @@ def test_attention_lora_rows(gpu, T, off, H, KV, kind, rot):
 
 
 # (T, off, H, KV): a decode step, 8 verify rows (prep_kernel, then verify_kernel), a prefill (prep_kernel writes the
-# q scratch, flash_kernel, the rotation in place after it)
+# q scratch, prefill_hilo_kernel with split keys, the rotation in the merge)
 @pytest.mark.parametrize("T,off,H,KV", [(1, 2047, 16, 4), (8, 1000, 8, 2), (100, 300, 8, 2)])
 def test_layer_lora_rows(gpu, T, off, H, KV):
     """bn_attn_layer (the whole arm, rotated) with the LoRA rows: u from the call's own output, and vs the oracle."""

@@ -97,8 +97,8 @@ def test_prefill_kernel_rescale_on_late_dominant_key(pf, q16):
 
 @pytest.mark.parametrize("q16", [True, False])
 def test_prefill_kernel_matches_default_path(pf, gpu, q16):
-    """The prefill kernels and flash_kernel agree (each is within 2e-3 of the oracle; here they are compared
-    directly)."""
+    """The prefill kernels and the default path of a call this small (split key ranges) agree (each is within 2e-3 of
+    the oracle; here they are compared directly)."""
     torch, ctx1, ws1 = gpu
     inp = workload.layer(6300, T=160, off=96, H=8, KV=2)
     if q16:

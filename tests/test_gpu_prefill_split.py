@@ -12,7 +12,7 @@ from glimpse_language_amd import bonsai_attn as ba
 
 pytestmark = pytest.mark.gpu
 
-# a tile short of two q-tiles and one row past; ranges of one, two and three key tiles (unsplit, then split in two);
+# a row short of two q-tiles and one row past; ranges of one, two and three key tiles (unsplit, then split in two);
 # q-tiles with different numbers of splits; one kv head with more than 64 splits of one q-tile (the merge's second pass)
 # and with more than 64 q-tiles (the block index scan's second pass); a range that ends on a tile's edge
 SHAPES = [(63, 0, 8, 2), (65, 0, 8, 2), (66, 30, 8, 2), (96, 0, 16, 4), (100, 300, 8, 2), (65, 5000, 4, 1),

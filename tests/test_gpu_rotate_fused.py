@@ -7,8 +7,8 @@ Checked two ways on every case:
   - against the oracle: oracle attention, then oracle gate_rotate with the gate logits set to +inf (sigmoid = 1
     exactly, so the oracle rotates its already-gated output): max-abs 2e-3 and the same projected argmax.
 Cases cover each kernel that can finish a row: the decode split kernel (one split), the split merge (many
-splits), verify rows, prefill_kernel and prefill_hilo_kernel (in their epilogues), flash_kernel (rotated in place after it) and ragged
-batches.
+splits), verify rows, prefill_kernel and prefill_hilo_kernel (in their epilogues), the merge of split key ranges and
+ragged batches.
 """
 import numpy as np
 import pytest

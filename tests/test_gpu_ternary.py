@@ -3,9 +3,9 @@
 Every output is within workload.ternary_tolerance of the oracle: 2e-5 of the L2 norm of its K products (fp32 sums in
 another order differ by about 3e-6 of it; a path that rounded x to fp16 would be off by about 2.4e-4), and within the
 north-star max-abs 2e-3. Repeated calls are bit-identical. Cases cover each kernel: the VALU rows kernel (T = 1..4),
-the split-K MFMA kernel (T = 5..32, K split 8, 4 or 2 ways), the 128-token MFMA kernel (T > 32, partly empty token
-and row tiles), and for T > 32 with a workspace the split-once pair (tern_split_kernel + tern_pf_kernel), whose
-results must equal the in-place kernel's bit for bit; one to three matrices sharing x, add into y, LoRA, code 3 and
+the split-K MFMA kernel (T = 5..32, K split 8, 4 or 2 ways), and for T > 32 the digits kernels (partly empty token and
+row tiles) with x's digits made by every block or, with a workspace, once (tern_digits_kernel), whose results must be the
+same bit for bit; one to three matrices sharing x, add into y, LoRA, code 3 and
 strided rows.
 """
 import numpy as np
@@ -81,7 +81,7 @@ CASES = [
     (6, 768, (128,)),              # K split 4 ways (768 = 4 * 192)
     (16, 384, (64, 64, 64)),       # K split 2 ways (384 = 2 * 192)
     (12, 640, (128,)),             # K split 2 ways (640 = 2 * 320, scale groups straddle the halves)
-    (32, 2048, (512,)), (33, 256, (704,)),              # first 128-token tile: partly empty token and row tiles
+    (32, 2048, (512,)), (33, 256, (704,)),              # first digits tiles: partly empty token and row tiles
     (130, 2048, (512, 128, 128)), (300, 1024, (320,)),
     (1, 128, (64,)), (8, 128, (64,)), (40, 128, (128,)),   # K = 128: one scale group, one or two chunks
 ]
@@ -98,8 +98,9 @@ def test_ternary_matches_oracle(gpu, T, K, os):
     assert all(np.array_equal(a, b) for a, b in zip(got, again)), "repeat call not bit-identical"
 
 
-# T > 32 shapes for the split-once pair: a partial last token tile, K = 128 (two chunks, one scale group), K = 640
-# (ten chunks, odd scale-group count per row), a second row member straddling a 256-row block, the 4B q/k/v shape
+# T > 32 shapes with x's digits made once: a partial last token tile, K = 128 (one scale group: one of two wave groups has
+# none), K = 640 (odd scale-group count per row), a second row member straddling a block, the 4B q/k/v shape (32 x 256
+# blocks; in place 32 x 512), the others 32 x 128 blocks with two wave groups
 SPLIT_CASES = [(33, 256, (704,)), (40, 128, (128,)), (100, 640, (192, 64)), (130, 2048, (512, 128, 128)),
                (300, 1024, (320,)), (257, 2560, (8192, 1024, 1024))]
 
@@ -118,11 +119,10 @@ def test_ternary_split_once_matches_in_place(gpu, T, K, os):
 
 
 def test_ternary_split_once_large_grid(gpu):
-    """A split-once call whose grid of 64-token blocks exceeds three per CU (1,300 tokens x 10,240 rows: 840 blocks)
-    takes the 128-token blocks of tern_pf_kernel (two x tiles per block; 21 x tiles, so the last block has one and a
-    short one), the smaller shapes above the 64-token blocks: bit-identical to the in-place kernel, and the first 64
-    rows of each matrix checked against the oracle. Then the same with a few x values beyond fp16's range, in a token
-    of each x tile of one block and in the last token (the scaled pass over both of a block's x tiles)."""
+    """A call with more than two 32 x 256 blocks per CU (1,300 tokens x 10,240 rows) takes 64 x 256 blocks (two x tiles
+    each, the last short), in place 64 x 512: bit-identical, and the first 64 rows of each matrix checked against the
+    oracle. Then the same with a few x values far above the rest, in a token of each x tile of one block and in the last
+    token (their blocks' second set of digits, in both of a block's x tiles)."""
     torch, ctx, _ = gpu
     T, K, os = 1300, 2560, (8192, 1024, 1024)
     print(f"ternary split-once large grid T={T}", flush=True)
@@ -141,8 +141,8 @@ def test_ternary_split_once_large_grid(gpu):
 
 
 def test_ternary_workspace_with_unaligned_scales(gpu):
-    """A scale array that is only 2-byte aligned cannot be copied 4 bytes at a time: with a workspace the call then
-    takes the in-place kernel, with the same results."""
+    """A scale array that is only 2-byte aligned is read a scale at a time instead of four groups' at once: the same
+    results with and without a workspace."""
     torch, ctx, _ = gpu
     T, K, os = 70, 512, (128,)
     mats, x, _, _ = make_case(0x7600, T, K, os)
@@ -215,8 +215,9 @@ def test_ternary_one_matrix_without_lora(gpu):
 @pytest.mark.parametrize("T,K,os", [(1, 1024, (256,)), (8, 2560, (2560,)), (16, 384, (64, 64, 64)),
                                     (40, 512, (128,)), (300, 1024, (320, 64))])
 def test_ternary_inputs_beyond_fp16_range(gpu, T, K, os):
-    """x with values from 2^15 to 2e8 in a few tokens and chunks (the MFMA kernels stage x as fp16 hi/lo parts, whose
-    range ends at 65504: those tokens' chunks take the scaled pass). On the MFMA kernels (T >= 5) every output is
+    """x with values from 2^15 to 2e8 in a few tokens and chunks (T = 5..32 stages x as fp16 hi/lo parts, whose range ends
+    at 65504: those tokens' chunks take the scaled pass; beyond 32 tokens their blocks take a second set of digits). On
+    the MFMA kernels (T >= 5) every output is
     within the relative bound of the oracle's fp32 matmul, small values of the large tokens included; the rows kernel
     (T <= 4) follows the reference's decode arithmetic, whose cancellation adds a term in s sum |x|. The other tokens'
     outputs are unaffected. The north-star 2e-3 absolute bar is not applied: outputs here reach 1e7, where fp32 sums
